@@ -16,11 +16,22 @@
 // clusters of a layer are enumerated from the parent layer's near box: each
 // lane reads one parent's mask of non-empty children (written by the tree
 // build), and the children outside this layer's near box are queued in LDS.
-// Every 64 queued clusters are staged in LDS, and every lane then reads each
-// one back (a broadcast) to evaluate it at its own point.  Batches whose
-// clusters all have the current size skip the per-cluster size test, and
-// clusters that lie beyond the core radius by construction skip the core
-// test.
+// Every 64 queued clusters are staged in LDS.  A lane holds a row of four
+// points and the four lanes of a row take every fourth cluster each
+// (BrickRows), so an LDS read and a cluster's y and z terms serve four
+// points; the lanes' shares are summed when the layer ends.  Batches whose
+// clusters all have one size skip the per-cluster size test, and clusters
+// that lie beyond the core radius by construction skip the core test.
+//
+// With one point per lane the five 16-byte LDS reads of a cluster took the
+// LDS return path 40 of the CU's cycles per 64 interactions, more than their
+// arithmetic: 3.0 ms for the 1M-vorton walk (129^3 points, near_k 3) and 3.5
+// ms for 256 effects of 33^3 (near_k 2).  With four they take 10 and the walk
+// is bound by VALU issue (23 operations per far interaction, about 3 cycles
+// each at the four waves per SIMD that its 101 registers allow): 1.89 and 2.5
+// ms.  Capping the registers at 96 or 80 for more waves was slower (2.9 ms
+// against 2.7 for the whole frame): the four points' interleaved chains hide
+// latency better than more waves do.
 #include "vg_internal.h"
 
 namespace vg {
@@ -46,12 +57,15 @@ __device__ __forceinline__ uint32_t layer_scale(const TreeView &tv, int l, int a
     return s;
 }
 
+// Children a parent may queue per round, and entries of the far-cluster queue.
+constexpr uint32_t kTake = 8, kQueue = 64 + 64 * kTake;
+
 // Per-wave LDS staging area: 64 fetched clusters (or vortons) at a time.
 struct WaveStage {
     float4 P[64], W[64], M0[64], M1[64], M2[64];
     // leaf row tables (offsets in [0, 64), starts in [64, 128)), or the
     // cluster queue of the layers above
-    uint32_t rows[128];
+    uint32_t rows[kQueue];
 };
 
 // Lane-strided walk over the cells of a bx x by x bz box: lane `lane` visits
@@ -100,68 +114,122 @@ struct SizeFactors {
     float size = -1.0f, r2 = 0.f, s = 0.f, ir3 = 0.f;
 };
 
-__device__ __forceinline__ void set_size(SizeFactors &f, float size, float spread, float3 &part,
-                                         float3 &scaled) {
-    scaled.x += part.x * f.s;
-    scaled.y += part.y * f.s;
-    scaled.z += part.z * f.s;
-    part = make_float3(0.f, 0.f, 0.f);
+__device__ __forceinline__ SizeFactors size_factors(float size, float spread) {
+    SizeFactors f;
     f.size = size;
     const float radius = size * 0.5f * spread;
     f.r2 = radius * radius;
     f.s = (2.0f / 3.0f) * f.r2 * radius;
     f.ir3 = __builtin_amdgcn_rcpf(f.r2 * radius);
+    return f;
 }
 
-// Monopole (+ first-moment) contribution of one cluster, unscaled by s.
-// m0..m2 carry the first moment's rows times 3 (.xyz, staged so by the
-// walk) and its antisymmetric part (.w, unscaled).
+// A lane's share of a brick: the four points x0..x0+3 of one (y, z) row.
+// The four lanes of a quad own the same row and take every fourth item
+// (cluster or vorton) each, so an item's LDS reads and its y and z terms
+// serve four points of a lane.
+struct Row4 {
+    float x[4], y, z;
+};
+struct Part4 {
+    float x[4], y[4], z[4];
+};
+
+__device__ __forceinline__ void part_clear(Part4 &p) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) p.x[i] = p.y[i] = p.z[i] = 0.f;
+}
+
+// DPP exchange inside a quad: lane ^ 1 (0xB1) or lane ^ 2 (0x4E).
+template <int CTRL>
+__device__ __forceinline__ float quad_swap(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+// The quad's four shares of four points summed so that lane l keeps point
+// l & 3: each step sends the half of the points it gives up.
+__device__ __forceinline__ float quad_own(const float v[4], uint32_t lane) {
+    const bool hi2 = (lane & 2u) != 0u, hi1 = (lane & 1u) != 0u;
+    const float a = (hi2 ? v[2] : v[0]) + quad_swap<0x4E>(hi2 ? v[0] : v[2]);
+    const float b = (hi2 ? v[3] : v[1]) + quad_swap<0x4E>(hi2 ? v[1] : v[3]);
+    return (hi1 ? b : a) + quad_swap<0xB1>(hi1 ? a : b);
+}
+
+// Adds the quad's shares times scale to the lane's own point and clears them.
+__device__ __forceinline__ void part_flush(Part4 &p, float scale, float3 &own, uint32_t lane) {
+    own.x += quad_own(p.x, lane) * scale;
+    own.y += quad_own(p.y, lane) * scale;
+    own.z += quad_own(p.z, lane) * scale;
+    part_clear(p);
+}
+
+// Monopole (+ first-moment) contribution of one cluster to a row's four
+// points, unscaled by s (SCALED: times f.s).  m0..m2 carry the first
+// moment's rows times 3 (.xyz, staged so by the walk) and its antisymmetric
+// part (.w, unscaled).
 // FAR: the caller knows the cluster lies outside the core radius (the law
 // inside the core never applies); d2 carries 1e-24 so that a cluster of
 // zero vorticity (whose centroid defaults to the origin) adds 0 even at a
 // query point on the origin (1e-24 is below half an ulp of any squared
 // distance above 1e-16, so elsewhere it can only settle a rounding tie).
-template <int POLICY, int ORDER, bool FAR = false>
-__device__ __forceinline__ void cluster_term(float3 &part, float3 q, float4 p, float4 w, float4 m0,
-                                             float4 m1, float4 m2, const SizeFactors &f) {
-    const float dx = q.x - p.x, dy = q.y - p.y, dz = q.z - p.z;
-    const float d2 = FAR ? fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, 1e-24f)))
-                         : dx * dx + dy * dy + dz * dz;
-    float law, rs2;
-    if (POLICY == VG_RSQRT_REFERENCE) {
-        rs2 = __builtin_amdgcn_rcpf(d2);
-        law = finvsqrtf(d2) * rs2;
-    } else {
-        const float rs = __builtin_amdgcn_rsqf(d2);
-        rs2 = rs * rs;
-        law = rs2 * rs;
-    }
-    const bool inside = !FAR && d2 < f.r2;
-    const float lm = inside ? f.ir3 : law;
-    if (ORDER >= 1) {
-        // (w x d) lm - (a - 3 rs2 (t x d)) ld with t = D d folds into
-        // ((w + c3 t3) x d) lm - a ld with t3 = 3 D d, c3 = rs2 outside the
-        // core, 0 inside (where ld = 0): one cross product instead of two
-        const float tx = m0.x * dx + m0.y * dy + m0.z * dz;
-        const float ty = m1.x * dx + m1.y * dy + m1.z * dz;
-        const float tz = m2.x * dx + m2.y * dy + m2.z * dz;
-        const float c3 = inside ? 0.0f : rs2;
-        const float vx = w.x + c3 * tx, vy = w.y + c3 * ty, vz = w.z + c3 * tz;
-        if (FAR) {
-            // lm = ld = law: ((v x d) - a) law, three fused operations a row
-            part.x = fmaf(fmaf(vy, dz, -fmaf(vz, dy, m0.w)), law, part.x);
-            part.y = fmaf(fmaf(vz, dx, -fmaf(vx, dz, m1.w)), law, part.y);
-            part.z = fmaf(fmaf(vx, dy, -fmaf(vy, dx, m2.w)), law, part.z);
+//
+// One point takes 18 VALU operations and an rsq with first moments (9 and
+// an rsq without); the y and z parts of the distance, of D d and of the
+// cross products are formed once for the four points.
+template <int POLICY, int ORDER, bool FAR, bool SCALED>
+__device__ __forceinline__ void cluster_row(Part4 &part, const Row4 &q, float4 p, float4 w,
+                                            float4 m0, float4 m1, float4 m2,
+                                            const SizeFactors &f) {
+    const float dy = q.y - p.y, dz = q.z - p.z;
+    const float dyz = FAR ? fmaf(dz, dz, fmaf(dy, dy, 1e-24f)) : fmaf(dz, dz, dy * dy);
+    // D d without its x term
+    const float t0 = fmaf(m0.z, dz, m0.y * dy), t1 = fmaf(m1.z, dz, m1.y * dy),
+                t2 = fmaf(m2.z, dz, m2.y * dy);
+    // w x d without its x terms
+    const float cx = fmaf(w.y, dz, -(w.z * dy)), cy = w.x * dz, cz = w.x * dy;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float dx = q.x[i] - p.x;
+        const float d2 = fmaf(dx, dx, dyz);
+        float law, rs2;
+        if (POLICY == VG_RSQRT_REFERENCE) {
+            rs2 = __builtin_amdgcn_rcpf(d2);
+            law = finvsqrtf(d2) * rs2;
         } else {
-            const float ld = inside ? 0.0f : law;
-            part.x += (vy * dz - vz * dy) * lm - m0.w * ld;
-            part.y += (vz * dx - vx * dz) * lm - m1.w * ld;
-            part.z += (vx * dy - vy * dx) * lm - m2.w * ld;
+            const float rs = __builtin_amdgcn_rsqf(d2);
+            rs2 = rs * rs;
+            law = rs2 * rs;
         }
-    } else {
-        part.x += (w.y * dz - w.z * dy) * lm;
-        part.y += (w.z * dx - w.x * dz) * lm;
-        part.z += (w.x * dy - w.y * dx) * lm;
+        const bool inside = !FAR && d2 < f.r2;
+        float lm = inside ? f.ir3 : law;
+        if (SCALED) lm *= f.s;
+        if (ORDER >= 1) {
+            // (w x d) lm - (a - 3 rs2 (t x d)) ld with t = D d folds into
+            // ((w + c3 t3) x d) lm - a ld with t3 = 3 D d, c3 = rs2 outside
+            // the core, 0 inside (where ld = 0): one cross product
+            const float c3 = inside ? 0.0f : rs2;
+            const float vx = fmaf(c3, fmaf(m0.x, dx, t0), w.x);
+            const float vy = fmaf(c3, fmaf(m1.x, dx, t1), w.y);
+            const float vz = fmaf(c3, fmaf(m2.x, dx, t2), w.z);
+            if (FAR) {
+                // lm = ld: ((v x d) - a) lm, three fused operations a row
+                part.x[i] = fmaf(fmaf(vy, dz, -fmaf(vz, dy, m0.w)), lm, part.x[i]);
+                part.y[i] = fmaf(fmaf(vz, dx, -fmaf(vx, dz, m1.w)), lm, part.y[i]);
+                part.z[i] = fmaf(fmaf(vx, dy, -fmaf(vy, dx, m2.w)), lm, part.z[i]);
+            } else {
+                const float ld = inside ? 0.0f : lm;
+                part.x[i] += (vy * dz - vz * dy) * lm - m0.w * ld;
+                part.y[i] += (vz * dx - vx * dz) * lm - m1.w * ld;
+                part.z[i] += (vx * dy - vy * dx) * lm - m2.w * ld;
+            }
+        } else {
+            part.x[i] = fmaf(cx, lm, part.x[i]);
+            part.y[i] = fmaf(fmaf(w.z, dx, -cy), lm, part.y[i]);
+            part.z[i] = fmaf(fmaf(-w.y, dx, cz), lm, part.z[i]);
+        }
+        // the rarely taken forms finish one point before the next: four
+        // interleaved ones would set the kernel's register count
+        if (ORDER >= 1 && !FAR) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -291,80 +359,213 @@ __device__ __forceinline__ float3 expansion_eval(Expansion &E, float3 x) {
     return make_float3(u[0], u[1], u[2]);
 }
 
-// One wave evaluates one brick of grid points; S is the wave's LDS slot.
-// Appends to the LDS queue Q (128 entries, qn < 64 on entry) the non-empty
-// cells of layer l that are children of the cells lo..hi of layer l + 1 and
-// lie outside the near box n0..n1, as tag | offset.  Each lane takes one
-// parent and reads its mask of non-empty children (so empty and near cells
-// are never loaded); the wave then appends one child per lane per round.
-// Whenever 64 entries are queued, flush() consumes Q[0, 64) and the rest
-// moves down.
-template <class Flush>
-__device__ __forceinline__ void queue_far_children(const TreeView &tv, int l, const int lo[3],
-                                                   const int hi[3], const int n0[3],
-                                                   const int n1[3], uint32_t tag,
-                                                   uint32_t *Q, uint32_t &qn, uint32_t lane,
-                                                   Flush &&flush) {
+// Inclusive sum over the wave: DPP shifts within rows of 16 lanes, then the
+// last lane of each row (pair of rows) broadcast to the next.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_add(uint32_t v) {
+    return v + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+    v = dpp_add<0x111, 0xf>(v);  // row_shr:1
+    v = dpp_add<0x112, 0xf>(v);  // row_shr:2
+    v = dpp_add<0x114, 0xf>(v);  // row_shr:4
+    v = dpp_add<0x118, 0xf>(v);  // row_shr:8
+    v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    v = dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+// Enumerates the non-empty cells of layer l that are children of the cells
+// lo..hi of layer l + 1 and lie outside the near box n0..n1, through the LDS
+// queue Q (kQueue entries).  Each lane takes one parent and reads its mask of
+// non-empty children (so empty and near cells are never loaded); a wave scan
+// of the counts gives each lane the slots of its children, up to kTake of
+// them per round (one scan per round instead of one ballot per child).
+// consume(first, count) then takes every full batch of 64 cell offsets from
+// Q[first], the last batch of the layer as it is.
+template <class Consume>
+__device__ __forceinline__ void far_children(const TreeView &tv, int l, const int lo[3],
+                                             const int hi[3], const int n0[3], const int n1[3],
+                                             uint32_t *Q, uint32_t lane, Consume &&consume) {
+    uint32_t qn = 0;  // entries waiting, fewer than 64 between rounds
     const vg_grid_desc &gl = tv.layer[l], &gp = tv.layer[l + 1];
     const uint32_t *__restrict__ Cm = tv.C[l + 1];
     const int dx = (int)tv.dec[l + 1][0], dy = (int)tv.dec[l + 1][1];
     const int dz = (int)tv.dec[l + 1][2];
+    const bool halves = dx == 2 && dy == 2 && dz == 2;
+    const uint32_t sy = gl.np[0], sz = gl.np[0] * gl.np[1];
     const int px = hi[0] - lo[0] + 1, py = hi[1] - lo[1] + 1, pz = hi[2] - lo[2] + 1;
     const int ptotal = px * py * pz;
     BoxIter it = box_begin(px, py, lane);
-    for (int base = 0; base < ptotal; base += 64, box_next(it)) {
-        uint32_t m = 0u, cbase = 0u;
-        if (it.z < pz) {
-            const int ax = lo[0] + it.x, ay = lo[1] + it.y, az = lo[2] + it.z;
-            m = Cm[cell_offset(gp, ax, ay, az)];
-            const int cx = ax * dx, cy = ay * dy, cz = az * dz;
-            cbase = cell_offset(gl, cx, cy, cz);
-            // children of this parent inside the near box, per axis (a
-            // decimation is at most 3)
-            uint32_t nx = 0u, ny = 0u, nz = 0u;
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                if (i < dx && cx + i >= n0[0] && cx + i <= n1[0]) nx |= 1u << i;
-                if (i < dy && cy + i >= n0[1] && cy + i <= n1[1]) ny |= 1u << i;
-                if (i < dz && cz + i >= n0[2] && cz + i <= n1[2]) nz |= 1u << i;
+    uint32_t m = 0u, cbase = 0u;
+    int base = 0;
+    for (;;) {
+        bool last = false;
+        while (__ballot(m != 0u) == 0ull) {  // the next 64 parents
+            if (base >= ptotal) {
+                last = true;
+                break;
             }
-            if (nx && ny && nz) {
-                uint32_t nm = 0u;
+            if (it.z < pz) {
+                const int ax = lo[0] + it.x, ay = lo[1] + it.y, az = lo[2] + it.z;
+                m = Cm[cell_offset(gp, ax, ay, az)];
+                const int cx = ax * dx, cy = ay * dy, cz = az * dz;
+                cbase = cell_offset(gl, cx, cy, cz);
+                if (halves) {
+                    // bits of the children on the low and high side of each axis
+                    // that lie inside the near box
+                    const uint32_t nx = (cx >= n0[0] && cx <= n1[0] ? 0x55u : 0u) |
+                                        (cx + 1 >= n0[0] && cx + 1 <= n1[0] ? 0xaau : 0u);
+                    const uint32_t ny = (cy >= n0[1] && cy <= n1[1] ? 0x33u : 0u) |
+                                        (cy + 1 >= n0[1] && cy + 1 <= n1[1] ? 0xccu : 0u);
+                    const uint32_t nz = (cz >= n0[2] && cz <= n1[2] ? 0x0fu : 0u) |
+                                        (cz + 1 >= n0[2] && cz + 1 <= n1[2] ? 0xf0u : 0u);
+                    m &= ~(nx & ny & nz);
+                } else {
+                    // children of this parent inside the near box, per axis (a
+                    // decimation is at most 3)
+                    uint32_t nx = 0u, ny = 0u, nz = 0u;
 #pragma unroll
-                for (int k = 0; k < 3; ++k)
+                    for (int i = 0; i < 3; ++i) {
+                        if (i < dx && cx + i >= n0[0] && cx + i <= n1[0]) nx |= 1u << i;
+                        if (i < dy && cy + i >= n0[1] && cy + i <= n1[1]) ny |= 1u << i;
+                        if (i < dz && cz + i >= n0[2] && cz + i <= n1[2]) nz |= 1u << i;
+                    }
+                    if (nx && ny && nz) {
+                        uint32_t nm = 0u;
 #pragma unroll
-                    for (int j = 0; j < 3; ++j)
-                        if (((nz >> k) & (ny >> j) & 1u) != 0u) nm |= nx << (dx * (j + dy * k));
-                m &= ~nm;
+                        for (int k = 0; k < 3; ++k)
+#pragma unroll
+                            for (int j = 0; j < 3; ++j)
+                                if (((nz >> k) & (ny >> j) & 1u) != 0u)
+                                    nm |= nx << (dx * (j + dy * k));
+                        m &= ~nm;
+                    }
+                }
             }
+            base += 64;
+            box_next(it);
         }
-        for (;;) {
-            const bool take = m != 0u;
-            const unsigned long long b = __ballot(take);
-            if (b == 0ull) break;
-            if (take) {
-                const uint32_t bit = (uint32_t)__builtin_ctz(m);
-                m &= m - 1u;
-                const uint32_t i = bit % (uint32_t)dx, jk = bit / (uint32_t)dx;
-                const uint32_t j = jk % (uint32_t)dy, k = jk / (uint32_t)dy;
-                const uint32_t below = (uint32_t)__popcll(b & ((1ull << lane) - 1ull));
-                Q[qn + below] = tag | (cbase + i + gl.np[0] * (j + gl.np[1] * k));
+        if (!last) {
+            const uint32_t c = min((uint32_t)__popc(m), kTake);
+            const uint32_t incl = wave_scan(c);
+            uint32_t at = qn + incl - c;
+#pragma unroll
+            for (uint32_t i = 0; i < kTake; ++i) {
+                if (i < c) {
+                    const uint32_t bit = (uint32_t)__builtin_ctz(m);
+                    m &= m - 1u;
+                    uint32_t off;
+                    if (halves) {
+                        off = cbase + (bit & 1u) + ((bit & 2u) ? sy : 0u) + ((bit & 4u) ? sz : 0u);
+                    } else {
+                        const uint32_t jk = bit / (uint32_t)dx, k = jk / (uint32_t)dy;
+                        off = cbase + (bit - jk * (uint32_t)dx) + (jk - k * (uint32_t)dy) * sy +
+                              k * sz;
+                    }
+                    Q[at++] = off;
+                }
             }
-            qn += (uint32_t)__popcll(b);
-            if (qn >= 64u) {
-                __builtin_amdgcn_wave_barrier();
-                flush();
-                const uint32_t rest = qn - 64u;
-                const uint32_t moved = lane < rest ? Q[64 + lane] : 0u;
-                __builtin_amdgcn_wave_barrier();
-                if (lane < rest) Q[lane] = moved;
-                __builtin_amdgcn_wave_barrier();
-                qn = rest;
-            }
+            qn += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        }
+        uint32_t first = 0;
+        if (qn >= (last ? 1u : 64u)) {
+            __builtin_amdgcn_wave_barrier();
+            do {
+                const uint32_t cnt = min(64u, qn - first);
+                consume(first, cnt);
+                first += cnt;
+            } while (first + (last ? 1u : 64u) <= qn);
+        }
+        if (last) break;
+        if (first) {
+            const uint32_t rest = qn - first;
+            const uint32_t moved = lane < rest ? Q[first + lane] : 0u;
+            __builtin_amdgcn_wave_barrier();
+            if (lane < rest) Q[lane] = moved;
+            __builtin_amdgcn_wave_barrier();
+            qn = rest;
         }
     }
 }
 
+// The points of one brick as the lanes of its wave hold them.  A row is the
+// four points of a brick along its row axis `ax`; the row axis is the first
+// one whose four points all exist (a brick at the grid's upper faces has
+// fewer on some axes), and the other two axes follow it cyclically, which
+// keeps the sense of the cross products.  A row's lanes (4, 16 or 64 of
+// them, as few rows allow) take the items of a batch in turn.
+struct BrickRows {
+    uint32_t ax, ay, az;  // grid axes of the rotated x, y, z
+    uint32_t slots;       // lanes per row
+    uint32_t slot;        // this lane's
+    Row4 q;               // this lane's row, rotated axes
+    uint32_t pt[3];       // the lane's own point, grid axes
+    bool owner;           // the lane writes its own point
+};
+
+__device__ __forceinline__ BrickRows brick_rows(const vg_grid_desc &g, const uint32_t bb[3],
+                                                uint32_t lane) {
+    uint32_t nv[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) nv[a] = min(4u, g.np[a] - 4 * bb[a]);
+    BrickRows r;
+    r.ax = nv[0] == 4u ? 0u : nv[1] == 4u ? 1u : nv[2] == 4u ? 2u : 0u;
+    r.ay = r.ax == 2u ? 0u : r.ax + 1u;
+    r.az = r.ay == 2u ? 0u : r.ay + 1u;
+    auto pick = [](const uint32_t v[3], uint32_t a) { return a == 0u ? v[0] : a == 1u ? v[1] : v[2]; };
+    const uint32_t nx = pick(nv, r.ax), ny = pick(nv, r.ay), nz = pick(nv, r.az);
+    const uint32_t rows = ny * nz;
+    r.slots = rows == 1u ? 64u : rows <= 4u ? 16u : 4u;
+    r.slot = lane & (r.slots - 1u);
+    uint32_t row = rows == 1u ? 0u : rows <= 4u ? lane >> 4 : lane >> 2;
+    const bool live = row < rows;
+    if (!live) row = rows - 1u;
+    const uint32_t jz = row / ny, jy = row - jz * ny;
+    const uint32_t jx = r.slot & 3u;
+    r.owner = live && r.slot < 4u && jx < nx;
+    const uint32_t b0[3] = {4 * bb[0], 4 * bb[1], 4 * bb[2]};
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t ix = min(i, nx - 1u);
+        uint32_t p[3];
+#pragma unroll
+        for (uint32_t a = 0; a < 3; ++a) p[a] = b0[a] + (a == r.ax ? ix : a == r.ay ? jy : jz);
+        const float3 c = grid_query_point(g, p[0], p[1], p[2]);
+        const float cv[3] = {c.x, c.y, c.z};
+        r.q.x[i] = r.ax == 0u ? cv[0] : r.ax == 1u ? cv[1] : cv[2];
+        r.q.y = r.ay == 0u ? cv[0] : r.ay == 1u ? cv[1] : cv[2];
+        r.q.z = r.az == 0u ? cv[0] : r.az == 1u ? cv[1] : cv[2];
+        if (i == min(jx, nx - 1u)) {
+#pragma unroll
+            for (int a = 0; a < 3; ++a) r.pt[a] = p[a];
+        }
+    }
+    return r;
+}
+
+// (x, y, z) with x moved to the row axis: component ax first.
+__device__ __forceinline__ float4 rotate(float4 v, uint32_t ax) {
+    if (ax == 0u) return v;
+    return ax == 1u ? make_float4(v.y, v.z, v.x, v.w) : make_float4(v.z, v.x, v.y, v.w);
+}
+// ... and back.
+__device__ __forceinline__ float3 rotate_back(float3 v, uint32_t ax) {
+    if (ax == 0u) return v;
+    return ax == 1u ? make_float3(v.z, v.x, v.y) : make_float3(v.y, v.z, v.x);
+}
+
+// Sum over a row's lanes beyond the quad (16 or 64 lanes per row).
+__device__ __forceinline__ float3 row_sum(float3 v, uint32_t slots) {
+    for (uint32_t m = 4u; m < slots; m <<= 1) {
+        v.x += __shfl_xor(v.x, (int)m, 64);
+        v.y += __shfl_xor(v.y, (int)m, 64);
+        v.z += __shfl_xor(v.z, (int)m, 64);
+    }
+    return v;
+}
+
+// One wave evaluates one brick of grid points; S is the wave's LDS slot.
 template <int POLICY, int ORDER, int COUNT>
 __device__ __forceinline__ void mac_brick(const TreeView &tv, const vg_grid_desc &g,
                                           const MacParams &mp, uint32_t brick, WaveStage &S,
@@ -373,15 +574,9 @@ __device__ __forceinline__ void mac_brick(const TreeView &tv, const vg_grid_desc
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t bb[3] = {brick % mp.nb[0], (brick / mp.nb[0]) % mp.nb[1],
                             brick / (mp.nb[0] * mp.nb[1])};
-    const uint32_t lp[3] = {lane & 3u, (lane >> 2) & 3u, lane >> 4};
-    uint32_t pt[3];
-    bool valid = true;
     int cl0[3], cl1[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        const uint32_t p = 4 * bb[a] + lp[a];
-        valid = valid && p < g.np[a];
-        pt[a] = p < g.np[a] ? p : g.np[a] - 1;
         const int nc = (int)g.np[a] - 1;
         const int first = (int)(4 * bb[a]);
         int last = first + 3;
@@ -389,7 +584,9 @@ __device__ __forceinline__ void mac_brick(const TreeView &tv, const vg_grid_desc
         cl0[a] = first < nc - 1 ? first : nc - 1;
         cl1[a] = last < nc - 1 ? last : nc - 1;
     }
-    const float3 q = grid_query_point(g, pt[0], pt[1], pt[2]);
+    const BrickRows br = brick_rows(g, bb, lane);
+    const Row4 &q = br.q;
+    const uint32_t slot = br.slot, slots = br.slots;
     float3 sum = make_float3(0.f, 0.f, 0.f), comp = sum;
     unsigned long long n_clusters = 0, n_pairs = 0, n_expand = 0;
     const bool expanding = mp.expand_from >= 1 && mp.expand_from <= (int)tv.depth - 2;
@@ -443,15 +640,19 @@ __device__ __forceinline__ void mac_brick(const TreeView &tv, const vg_grid_desc
                     }
                     n_expand += __popcll(__ballot(use));
                 }
-            } else if (l == mp.expand_from && valid) {
-                const size_t o = point_offset(g, pt[0], pt[1], pt[2]);
-                kahan_add(sum, comp, make_float3(out[3 * o], out[3 * o + 1], out[3 * o + 2]));
+            } else if (l == mp.expand_from && br.owner) {
+                const size_t o = point_offset(g, br.pt[0], br.pt[1], br.pt[2]);
+                const float4 u =
+                    rotate(make_float4(out[3 * o], out[3 * o + 1], out[3 * o + 2], 0.f), br.ax);
+                kahan_add(sum, comp, make_float3(u.x, u.y, u.z));
             }
 #pragma unroll
             for (int a = 0; a < 3; ++a) { lo[a] = n0[a]; hi[a] = n1[a]; }
             continue;
         }
-        float3 part = make_float3(0.f, 0.f, 0.f), scaled = part;
+        Part4 part;
+        part_clear(part);
+        float3 own = make_float3(0.f, 0.f, 0.f);
         if (COUNT) {
             BoxIter it = box_begin(bx, by, lane);
             for (int base = 0; base < total; base += 64, box_next(it)) {
@@ -468,13 +669,14 @@ __device__ __forceinline__ void mac_brick(const TreeView &tv, const vg_grid_desc
             // Far clusters of the layer come through the LDS queue, 64 at a
             // time (fewer than 64 wait between rounds).
             uint32_t *Q = S.rows;
-            uint32_t qn = 0;
-            auto consume = [&](uint32_t cnt) {
+            auto consume = [&](uint32_t first, uint32_t cnt) {
+                // lanes past the count stage the first cluster's position
+                // with zero vorticity: they add nothing
                 const bool use = lane < cnt;
-                const uint32_t off = use ? Q[lane] : 0u;
-                float4 p = make_float4(0.f, 0.f, 0.f, 0.f), w = p, m0 = p, m1 = p, m2 = p;
+                const uint32_t off = Q[first + (use ? lane : 0u)];
+                const float4 p = P[off];
+                float4 w = make_float4(0.f, 0.f, 0.f, 0.f), m0 = w, m1 = w, m2 = w;
                 if (use) {
-                    p = P[off];
                     w = W[off];
                     if (ORDER) {
                         m0 = M[3 * (size_t)off];
@@ -482,73 +684,55 @@ __device__ __forceinline__ void mac_brick(const TreeView &tv, const vg_grid_desc
                         m2 = M[3 * (size_t)off + 2];
                     }
                 }
-                unsigned long long mask = __ballot(use);
-                S.P[lane] = p;
-                S.W[lane] = w;
+                S.P[lane] = rotate(p, br.ax);
+                S.W[lane] = rotate(w, br.ax);
                 if (ORDER) {
-                    // rows times 3 (cluster_term's convention), once per cluster
+                    if (br.ax != 0u) {
+                        const float4 r0 = rotate(m0, br.ax), r1 = rotate(m1, br.ax),
+                                     r2 = rotate(m2, br.ax);
+                        m0 = br.ax == 1u ? r1 : r2;
+                        m1 = br.ax == 1u ? r2 : r0;
+                        m2 = br.ax == 1u ? r0 : r1;
+                    }
+                    // rows times 3 (cluster_row's convention), once per cluster
                     S.M0[lane] = make_float4(3.0f * m0.x, 3.0f * m0.y, 3.0f * m0.z, m0.w);
                     S.M1[lane] = make_float4(3.0f * m1.x, 3.0f * m1.y, 3.0f * m1.z, m1.w);
                     S.M2[lane] = make_float4(3.0f * m2.x, 3.0f * m2.y, 3.0f * m2.z, m2.w);
                 }
-                // every cluster of the batch has the current size (the usual
-                // case: one vorton size per tree)?
-                const bool one_size = __ballot(use && p.w != f.size) == 0ull;
+                // the batch's clusters have one size (the usual case: one
+                // vorton size per tree)?
+                const float size = __int_as_float((int)uni((uint32_t)__float_as_int(p.w)));
+                const bool one_size = __ballot(p.w != size) == 0ull;
+                if (!one_size || size != f.size) {
+                    part_flush(part, f.s, own, lane);
+                    f = size_factors(size, spread);
+                }
                 __builtin_amdgcn_wave_barrier();
+                const uint32_t steps = (cnt + slots - 1u) / slots;  // one cluster per slot a step
                 if (one_size && f.r2 < far2) {
-                    // no size test (the five LDS reads of a cluster go out
-                    // together, one wait per cluster), and no core test
-                    while (mask) {
-                        const int j = __builtin_ctzll(mask);
-                        mask &= mask - 1;
-                        const float4 cp = S.P[j], cw = S.W[j];
-                        float4 a0 = cp, a1 = cp, a2 = cp;
-                        if (ORDER) {
-                            a0 = S.M0[j];
-                            a1 = S.M1[j];
-                            a2 = S.M2[j];
-                        }
-                        cluster_term<POLICY, ORDER, true>(part, q, cp, cw, a0, a1, a2, f);
-                    }
-                } else if (one_size) {
-                    while (mask) {
-                        const int j = __builtin_ctzll(mask);
-                        mask &= mask - 1;
-                        const float4 cp = S.P[j], cw = S.W[j];
-                        float4 a0 = cp, a1 = cp, a2 = cp;
-                        if (ORDER) {
-                            a0 = S.M0[j];
-                            a1 = S.M1[j];
-                            a2 = S.M2[j];
-                        }
-                        cluster_term<POLICY, ORDER>(part, q, cp, cw, a0, a1, a2, f);
-                    }
+                    for (uint32_t k = 0, j = slot; k < steps; ++k, j += slots)
+                        cluster_row<POLICY, ORDER, true, false>(part, q, S.P[j], S.W[j], S.M0[j],
+                                                                S.M1[j], S.M2[j], f);
                 } else {
-                    while (mask) {
-                        const int j = __builtin_ctzll(mask);
-                        mask &= mask - 1;
+                    // one size keeps part in units of s; several sizes scale
+                    // each cluster by its own
+                    SizeFactors fj = f;
+                    fj.s = 1.0f;
+                    for (uint32_t k = 0, j = slot; k < steps; ++k, j += slots) {
                         const float4 cp = S.P[j];
-                        if (cp.w != f.size) set_size(f, cp.w, spread, part, scaled);
-                        const float4 cw = S.W[j];
-                        float4 a0 = cp, a1 = cp, a2 = cp;
-                        if (ORDER) {
-                            a0 = S.M0[j];
-                            a1 = S.M1[j];
-                            a2 = S.M2[j];
-                        }
-                        cluster_term<POLICY, ORDER>(part, q, cp, cw, a0, a1, a2, f);
+                        if (!one_size) fj = size_factors(cp.w, spread);
+                        cluster_row<POLICY, ORDER, false, true>(part, q, cp, S.W[j], S.M0[j],
+                                                                S.M1[j], S.M2[j], fj);
                     }
+                    if (!one_size) part_flush(part, 1.0f, own, lane);
                 }
                 __builtin_amdgcn_wave_barrier();
             };
-            queue_far_children(tv, l, lo, hi, n0, n1, 0u, Q, qn, lane, [&] { consume(64u); });
+            far_children(tv, l, lo, hi, n0, n1, Q, lane, consume);
             __builtin_amdgcn_wave_barrier();
-            if (qn) consume(qn);
+            part_flush(part, f.s, own, lane);
         }
-        scaled.x += part.x * f.s;
-        scaled.y += part.y * f.s;
-        scaled.z += part.z * f.s;
-        kahan_add(sum, comp, scaled);
+        kahan_add(sum, comp, own);
 #pragma unroll
         for (int a = 0; a < 3; ++a) { lo[a] = n0[a]; hi[a] = n1[a]; }
     }
@@ -563,7 +747,9 @@ __device__ __forceinline__ void mac_brick(const TreeView &tv, const vg_grid_desc
         hi[2] = (int)g0.np[2] - 2;
     }
     {
-        float3 part = make_float3(0.f, 0.f, 0.f), scaled = part;
+        Part4 part;
+        part_clear(part);
+        float3 own = make_float3(0.f, 0.f, 0.f);
         const int ry = hi[1] - lo[1] + 1, rz = hi[2] - lo[2] + 1;
         const int nrows = ry * rz;
         for (int rbase = 0; rbase < nrows; rbase += 64) {
@@ -577,13 +763,8 @@ __device__ __forceinline__ void mac_brick(const TreeView &tv, const vg_grid_desc
                 rc = tv.cell_start[k1] + tv.cell_count[k1] - rs;
             }
             // inclusive scan of the row counts across the wave
-            uint32_t incl = rc;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const uint32_t tt = __shfl_up(incl, off, 64);
-                if ((int)lane >= off) incl += tt;
-            }
-            const uint32_t total = uni(__shfl(incl, 63, 64));
+            const uint32_t incl = wave_scan(rc);
+            const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
             if (COUNT) {
                 n_pairs += total;
                 continue;
@@ -592,50 +773,56 @@ __device__ __forceinline__ void mac_brick(const TreeView &tv, const vg_grid_desc
             S.rows[64 + lane] = rs;
             __builtin_amdgcn_wave_barrier();
             for (uint32_t vbase = 0; vbase < total; vbase += 64) {
-                const uint32_t t = vbase + lane;
-                float4 p = make_float4(0.f, 0.f, 0.f, 0.f), w = p;
-                if (t < total) {
-                    // last row whose offset is <= t
-                    int lo_i = 0, hi_i = 63;
-                    while (lo_i < hi_i) {
-                        const int mid = (lo_i + hi_i + 1) >> 1;
-                        if (S.rows[mid] <= t) lo_i = mid;
-                        else hi_i = mid - 1;
-                    }
-                    const uint32_t idx = S.rows[64 + lo_i] + (t - S.rows[lo_i]);
-                    p = tv.sorted_p[idx];
-                    w = tv.sorted_w[idx];
-                }
-                const bool one_size = __ballot(t < total && p.w != f.size) == 0ull;
-                __builtin_amdgcn_wave_barrier();
-                S.P[lane] = p;
-                S.W[lane] = w;
-                __builtin_amdgcn_wave_barrier();
+                // lanes past the count stage the first vorton's position with
+                // zero vorticity: they add nothing
                 const uint32_t cnt = total - vbase < 64u ? total - vbase : 64u;
+                const bool use = lane < cnt;
+                const uint32_t t = use ? vbase + lane : vbase;
+                // last row whose offset is <= t
+                int lo_i = 0, hi_i = 63;
+                while (lo_i < hi_i) {
+                    const int mid = (lo_i + hi_i + 1) >> 1;
+                    if (S.rows[mid] <= t) lo_i = mid;
+                    else hi_i = mid - 1;
+                }
+                const uint32_t idx = S.rows[64 + lo_i] + (t - S.rows[lo_i]);
+                const float4 p = tv.sorted_p[idx];
+                float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (use) w = tv.sorted_w[idx];
+                const float size = __int_as_float((int)uni((uint32_t)__float_as_int(p.w)));
+                const bool one_size = __ballot(p.w != size) == 0ull;
+                if (!one_size || size != f.size) {
+                    part_flush(part, f.s, own, lane);
+                    f = size_factors(size, spread);
+                }
+                __builtin_amdgcn_wave_barrier();
+                S.P[lane] = rotate(p, br.ax);
+                S.W[lane] = rotate(w, br.ax);
+                __builtin_amdgcn_wave_barrier();
+                const uint32_t steps = (cnt + slots - 1u) / slots;
                 if (one_size) {
-                    for (uint32_t j = 0; j < cnt; ++j) {
-                        const float4 vp = S.P[j], vw = S.W[j];
-                        cluster_term<POLICY, 0>(part, q, vp, vw, vp, vp, vp, f);
+                    for (uint32_t k = 0, j = slot; k < steps; ++k, j += slots) {
+                        const float4 vp = S.P[j];
+                        cluster_row<POLICY, 0, false, false>(part, q, vp, S.W[j], vp, vp, vp, f);
                     }
                 } else {
-                    for (uint32_t j = 0; j < cnt; ++j) {
+                    for (uint32_t k = 0, j = slot; k < steps; ++k, j += slots) {
                         const float4 vp = S.P[j];
-                        if (vp.w != f.size) set_size(f, vp.w, spread, part, scaled);
-                        cluster_term<POLICY, 0>(part, q, vp, S.W[j], vp, vp, vp, f);
+                        cluster_row<POLICY, 0, false, true>(part, q, vp, S.W[j], vp, vp, vp,
+                                                            size_factors(vp.w, spread));
                     }
+                    part_flush(part, 1.0f, own, lane);
                 }
                 __builtin_amdgcn_wave_barrier();
             }
         }
-        scaled.x += part.x * f.s;
-        scaled.y += part.y * f.s;
-        scaled.z += part.z * f.s;
-        kahan_add(sum, comp, scaled);
+        part_flush(part, f.s, own, lane);
+        kahan_add(sum, comp, own);
     }
     if (COUNT) {
         // the ballot must run on every lane: inside the lane-0 branch only
         // lane 0 would vote
-        const unsigned long long nv = (unsigned long long)__popcll(__ballot(valid));
+        const unsigned long long nv = (unsigned long long)__popcll(__ballot(br.owner));
         if (lane == 0) {
             atomicAdd(&counts[0], n_clusters * nv);
             atomicAdd(&counts[1], n_pairs * nv);
@@ -643,8 +830,9 @@ __device__ __forceinline__ void mac_brick(const TreeView &tv, const vg_grid_desc
         }
         return;
     }
-    if (valid) {
-        const size_t o = point_offset(g, pt[0], pt[1], pt[2]);
+    sum = rotate_back(row_sum(sum, slots), br.ax);
+    if (br.owner) {
+        const size_t o = point_offset(g, br.pt[0], br.pt[1], br.pt[2]);
         out[3 * o] = sum.x * mp.circ;
         out[3 * o + 1] = sum.y * mp.circ;
         out[3 * o + 2] = sum.z * mp.circ;
