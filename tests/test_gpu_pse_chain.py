@@ -1,0 +1,54 @@
+"""The viscous exchange's chain form (fractions precomputed, one component
+per workgroup) at the sizes where it changes: cells of one vorton up to more
+than two chunks of 64 lanes, a neighbourhood just within and just past the
+partners that fit a wave's LDS buffer, and slices that fit the LDS and that
+do not.  Bit for bit against the CPU oracle, with dead vortons."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+F32 = np.float32
+
+
+def run(vg, oracle, og, pos, om, size, rng, dead=0.15):
+    n = len(pos)
+    birth = np.where(rng.random(n) < dead, -1, 5).astype(np.int32)
+    dp, dw = vg.DeviceArray.from_numpy(pos), vg.DeviceArray.from_numpy(om)
+    db = vg.DeviceArray.from_numpy(birth)
+    t = vg.Tree()
+    t.build(vg.GridDesc.from_fields(og), vg.vortons_view(dp, dw, n, uniform_size=size))
+    t.pse_diffuse(dw, 0.5, 0.2, birth=db, birth_stride=1)
+    vg.synchronize()
+    want = oracle.pse_diffuse(og, pos, om, size, 0.5, 0.2, alive=birth >= 0)
+    assert np.array_equal(dw.numpy(), want)
+
+
+@pytest.mark.parametrize("blob", [1, 2, 3, 63, 64, 65, 127, 128, 129, 700, 2399, 2401])
+def test_chunks_of_here_vortons(vg, oracle, blob):
+    """One cell of `blob` vortons (its neighbours hold none) among cells of a
+    few."""
+    print(f"[case] PSE chain, a cell of {blob} vortons", flush=True)
+    rng = np.random.default_rng(blob)
+    cells, h = (8, 6, 5), 0.25
+    ext = np.array(cells) * h
+    pos = (rng.uniform(0.02, 0.98, (300, 3)) * ext)
+    around = np.all(np.abs(pos - np.array([4.5, 3.5, 2.5]) * h) < 1.6 * h, axis=1)
+    lump = (np.array([4, 3, 2]) + rng.uniform(0.1, 0.9, (blob, 3))) * h
+    pos = np.concatenate([pos[~around], lump]).astype(F32)
+    om = rng.normal(size=pos.shape).astype(F32)
+    og = oracle.define_shape(int(np.prod(cells)), np.zeros(3), ext, pow2=False)
+    assert og.shape == tuple(c + 1 for c in cells)
+    run(vg, oracle, og, pos, om, 0.2, rng)
+
+
+def test_slices_past_the_lds(vg, oracle):
+    """A thin slab: 50,000 vortons in two slices (200 KB a component)."""
+    print("[case] PSE chain, 100,000 vortons in a slab of four slices", flush=True)
+    rng = np.random.default_rng(9)
+    cells = (96, 96, 4)
+    ext = np.array(cells) * 0.02
+    pos = (rng.uniform(0.001, 0.999, (100000, 3)) * ext).astype(F32)
+    om = rng.normal(size=pos.shape).astype(F32)
+    og = oracle.define_shape(int(np.prod(cells)), np.zeros(3), ext, pow2=False)
+    assert og.shape == tuple(c + 1 for c in cells)
+    run(vg, oracle, og, pos, om, 0.02, rng)

@@ -23,14 +23,27 @@
 // (z, z+1), so each gets a workgroup; a barrier separates steps and a
 // launch separates the phases.  A step lasts as long as its busiest wave, so
 // k_pse_schedule first deals the non-empty cells of every step to the
-// waves, largest first, each to the least loaded wave.  The exchange
-// fraction f of a pair depends on positions and sizes only, so
-// k_pse_fractions computes those of the cells of 4+ vortons over the whole
-// chip beforehand, and their serial chains only move Omega.  The vorton
-// state lives in the tree's cell-sorted order (positions and sizes from the
-// tree, angular velocities gathered from the caller and scattered back), so
-// a cell's vortons are contiguous.  exp is vg_pse_exp, the same function as
-// the oracle's.
+// waves, largest first, each to the least loaded wave.
+//
+// A cell's exchanges are a serial chain, and the chains are what the call
+// waits for: 47k systolic steps (pse_cell_chain) in 540 cells on the slowest
+// slices of the two phases at 1M vortons (129^3), 16.5 ms when a step moved
+// all of Omega and its index down the lanes and stored through memory, 3.8
+// ms now.  So a step carries as little as it can:
+//   * the exchange fraction f of a pair depends on positions and sizes only:
+//     k_pse_fractions computes all of them over the whole chip beforehand, in
+//     the order the steps read them, with the step's other decisions (which
+//     lane exchanges, which adopts its own vorton) folded into f;
+//   * f is shared by the three components of Omega, which are otherwise
+//     independent: each has its own workgroup per slice (blockIdx.y);
+//   * a cell's partners wait in LDS, so a step is one lane shift and one
+//     exchange of one float.
+// The vorton state lives in the tree's cell-sorted order (positions and
+// sizes from the tree, angular velocities gathered from the caller and
+// scattered back), so a cell's vortons are contiguous.  exp is vg_pse_exp,
+// the same function as the oracle's.  Cells with more than kChainPartners
+// partners, or fractions that would fill 8 GB, take the form with the
+// fractions in the chain (k_pse_phase).
 #include <cstdlib>
 
 #include "vg_internal.h"
@@ -40,7 +53,16 @@ vg_status tree_checked_view(const vg_tree *t, TreeView *v);
 
 namespace {
 
-constexpr int kPseThreads = 512;
+constexpr int kPseThreads = 512;     // k_pse_phase
+constexpr int kChainThreads = 1024;  // k_pse_phase_chain (512: 4.5 against 4.0 ms)
+constexpr int kPseWaves = kPseThreads / 64, kChainWaves = kChainThreads / 64;
+// Vortons of a cell and its 7 forward cells that the chain's LDS buffers hold
+// (16 waves share 160 KB); 1M vortons at 129^3 have at most 442.
+constexpr uint32_t kChainPartners = 2400;
+// LDS floats of a wave's partner buffer besides the partners: up to 63 + 3
+// before them and up to 70 after (pse_cell_chain's out and in).
+constexpr uint32_t kBufFront = 68, kBufBack = 80;
+constexpr size_t kLdsBytes = 160 * 1024;  // of a CU
 
 // Cody-Waite reduction with the 16-bit split of ln 2, degree-7 Taylor
 // polynomial, 2^k from the exponent bits; 0 below -87.
@@ -91,11 +113,6 @@ struct PseArgs {
     const float4 *p;                // sorted (x, y, z, size)
     float4 *w;                      // sorted (Omega, alive)
     float nu_dt2, dissipation;
-    // Exchange fractions of the systolic cells, precomputed (or null): the
-    // cell with leaf point c holds frac[frac_off[c] + i n + j] for here-vorton
-    // i < k and partner j < n (0 where j <= i).
-    const float *frac;
-    const uint32_t *frac_off;
 };
 
 __device__ __forceinline__ void pse_cell(const PseArgs &a, uint32_t x, uint32_t y, uint32_t z) {
@@ -232,101 +249,6 @@ __device__ __forceinline__ void pse_cell_systolic(const PseArgs &a, const uint32
     }
 }
 
-// Lane l takes lane l + 1 (wrapping): the whole-wave DPP rotation
-// (wave_rol:1), so the window's next partner is always in lane 0.
-__device__ __forceinline__ float wave_rol(float v) {
-    return __int_as_float(
-        __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x134, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float4 wave_rol4(float4 v) {
-    return make_float4(wave_rol(v.x), wave_rol(v.y), wave_rol(v.z), wave_rol(v.w));
-}
-__device__ __forceinline__ uint32_t wave_rol_u(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x134, 0xf, 0xf, false);
-}
-__device__ __forceinline__ uint32_t wave_shr_u(uint32_t v, uint32_t in) {
-    return (uint32_t)__builtin_amdgcn_update_dpp((int)in, (int)v, 0x138, 0xf, 0xf, false);
-}
-
-// The systolic cell with its fractions read from a.frac: only Omega (and
-// its vorton's index, for the write-back of partners leaving the last lane)
-// streams down the lanes.  The window of 64 loaded partners rotates by one
-// lane per step, so lane 0 always holds the next partner to enter; each
-// lane's fractions are loaded kFracAhead steps before use (a lane walks its
-// row of the fraction block left to right).
-constexpr int kFracAhead = 8;
-
-__device__ __forceinline__ void pse_cell_systolic_frac(const PseArgs &a, uint32_t c,
-                                                       const uint32_t base[8],
-                                                       const uint32_t pre[9], uint32_t k,
-                                                       uint32_t n) {
-#pragma clang fp contract(off)
-    const int lane = (int)(threadIdx.x & 63);
-    const float *__restrict__ fc = a.frac + a.frac_off[c];
-    for (uint32_t B = 0; B < k; B += 64) {
-        const uint32_t L = k - B < 64u ? k - B : 64u;
-        const uint32_t i = B + (uint32_t)lane;
-        const uint32_t gi = base[0] + i;  // here-vortons are the cell's own
-        float4 wh = make_float4(0.f, 0.f, 0.f, 0.f), sw = wh, bw = wh;
-        uint32_t sg = 0, bg = 0;
-        bool live = false;
-        const uint32_t steps = (n - B) + L - 1;
-        // fraction of this lane at step t (0 unless it exchanges then)
-        auto fetch = [&](uint32_t t) -> float {
-            const int jl = (int)t - lane;
-            const uint32_t j = B + (uint32_t)jl;
-            return ((uint32_t)lane < L && jl > lane && j < n) ? fc[(size_t)i * n + j] : 0.f;
-        };
-        float cur[kFracAhead], nxt[kFracAhead];
-#pragma unroll
-        for (int d = 0; d < kFracAhead; ++d) cur[d] = fetch((uint32_t)d);
-        for (uint32_t t0 = 0; t0 < steps; t0 += kFracAhead) {
-#pragma unroll
-            for (int d = 0; d < kFracAhead; ++d) nxt[d] = fetch(t0 + kFracAhead + (uint32_t)d);
-#pragma unroll
-            for (int d = 0; d < kFracAhead; ++d) {
-                const uint32_t t = t0 + (uint32_t)d;
-                if (t >= steps) break;
-                if ((t & 63u) == 0) {  // the next 64 partners to enter, one per lane
-                    const uint32_t jj = B + t + (uint32_t)lane;
-                    if (jj < n) {
-                        bg = partner_index(base, pre, jj);
-                        bw = a.w[bg];
-                    }
-                }
-                sw = wave_shr4(sw, bw);  // lane 0 takes the window's lane 0
-                sg = wave_shr_u(sg, bg);
-                bw = wave_rol4(bw);
-                bg = wave_rol_u(bg);
-                const int jl = (int)t - lane;  // partner j - B at this lane
-                const uint32_t j = B + (uint32_t)jl;
-                if ((uint32_t)lane < L && jl >= 0 && j < n) {
-                    if (jl == lane) {  // j == i: the here-vorton itself
-                        wh = sw;
-                        live = sw.w != 0.f;
-                    } else if (jl > lane && live) {
-                        exchange_f(wh, sw, cur[d]);
-                    }
-                    if (j == n - 1) {  // the lane's last partner: done
-                        if (live) {
-                            wh.x -= wh.x * a.dissipation;
-                            wh.y -= wh.y * a.dissipation;
-                            wh.z -= wh.z * a.dissipation;
-                        }
-                        a.w[gi] = wh;
-                    }
-                    // a partner that is not a here-vorton of this chunk leaves
-                    // the last lane with its value for the next chunk
-                    if ((uint32_t)lane == L - 1 && j >= B + L) a.w[sg] = sw;
-                }
-            }
-#pragma unroll
-            for (int d = 0; d < kFracAhead; ++d) cur[d] = nxt[d];
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    }
-}
-
 __device__ __forceinline__ void pse_cell_wave(const PseArgs &a, uint32_t x, uint32_t y, uint32_t z) {
 #pragma clang fp contract(off)
     const int lane = (int)(threadIdx.x & 63);
@@ -343,10 +265,7 @@ __device__ __forceinline__ void pse_cell_wave(const PseArgs &a, uint32_t x, uint
     const uint32_t k = pre[1], n = pre[8];
     if (k == 0) return;
     if (k >= kSystolicMin) {
-        if (a.frac)
-            pse_cell_systolic_frac(a, c, base, pre, k, n);
-        else
-            pse_cell_systolic(a, base, pre, k, n);
+        pse_cell_systolic(a, base, pre, k, n);
         return;
     }
     if (n > 64u * kSlots) {
@@ -426,73 +345,260 @@ __device__ __forceinline__ void pse_cell_wave(const PseArgs &a, uint32_t x, uint
         if (G[s] >= 0) a.w[G[s]] = W[s];
 }
 
-// One workgroup per slice z = phase + 2 blockIdx.x (z < nz - 1); each wave
-// takes whole cells of the current wavefront step.
-constexpr int kPseWaves = kPseThreads / 64;
+__global__ void k_pse_zero64(unsigned long long *v) { v[threadIdx.x] = 0ull; }
 
-__global__ void k_pse_zero64(unsigned long long *v) { *v = 0ull; }
-
-// Fraction block size of each leaf point's cell (k n for systolic cells,
-// else 0), and the 64-bit total.
-__global__ __launch_bounds__(256) void k_pse_frac_size(PseArgs a, uint32_t cells,
-                                                       uint32_t *__restrict__ size,
-                                                       unsigned long long *__restrict__ total) {
-    __shared__ unsigned long long part[256];
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    unsigned long long kn = 0;
-    if (c < cells) {
-        const uint32_t k = a.count[c];
-        if (k >= kSystolicMin) {
-            const uint32_t nx = a.nx, nxy = a.nx * a.ny;
-            const uint32_t offs[8] = {0, 1, nx, 1 + nx, nxy, 1 + nxy, nx + nxy, 1 + nx + nxy};
-            uint32_t n = 0;
+// A cell's own vortons and those of its 7 forward cells, in partner order.
+struct CellPartners {
+    uint32_t base[8], pre[9];
+};
+__device__ __forceinline__ CellPartners cell_partners(const PseArgs &a, uint32_t c) {
+    const uint32_t nx = a.nx, nxy = a.nx * a.ny;
+    const uint32_t offs[8] = {0, 1, nx, 1 + nx, nxy, 1 + nxy, nx + nxy, 1 + nx + nxy};
+    CellPartners p;
+    p.pre[0] = 0;
 #pragma unroll
-            for (int r = 0; r < 8; ++r) n += a.count[c + offs[r]];
-            kn = (unsigned long long)k * n;
-        }
-        size[c] = kn < 0x80000000ull ? (uint32_t)kn : 0x80000000u;
+    for (int r = 0; r < 8; ++r) {
+        p.base[r] = a.start[c + offs[r]];
+        p.pre[r + 1] = p.pre[r] + a.count[c + offs[r]];
     }
-    part[threadIdx.x] = kn;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0 && part[0]) atomicAdd(total, part[0]);
+    return p;
 }
 
-// Exchange fractions of the systolic cells, one wave per leaf point's cell:
-// the same operations as the in-chain exchange, so the same bits.
+// The vortons of slices z and z + 1: contiguous in the cell-sorted order.
+struct SlicePair {
+    uint32_t first, count;
+};
+__device__ __forceinline__ SlicePair slice_pair(const PseArgs &a, uint32_t z, uint32_t n) {
+    const uint32_t nxy = a.nx * a.ny;
+    const uint32_t first = a.start[z * nxy];
+    return SlicePair{first, (z + 2 < a.nz ? a.start[(z + 2) * nxy] : n) - first};
+}
+
+// Systolic steps of the chunk of L here-vortons starting at B of a cell with
+// n partners, in groups of four (a lane reads four fractions at a time).
+__device__ __forceinline__ uint32_t chunk_groups(uint32_t n, uint32_t B, uint32_t L) {
+    return ((n - B) + L - 1 + 3) / 4;
+}
+
+// Fractions (floats) of each leaf point's cell, their 64-bit sum, the largest
+// partner count and the largest number of vortons in two adjacent slices
+// (totals[0..2]).  A grid-stride loop: with one workgroup per 256 points the
+// two atomics of each took 157 us at 129^3.
+__global__ __launch_bounds__(256) void k_pse_frac_size(PseArgs a, uint32_t cells, uint32_t n_all,
+                                                       uint32_t *__restrict__ size,
+                                                       unsigned long long *__restrict__ totals) {
+    __shared__ unsigned long long part[256];
+    __shared__ uint32_t most[256];
+    unsigned long long sum = 0;
+    uint32_t widest = 0;
+    for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < cells;
+         c += gridDim.x * blockDim.x) {
+        const uint32_t k = a.count[c];
+        unsigned long long f = 0;
+        if (k) {
+            const uint32_t n = cell_partners(a, c).pre[8];
+            for (uint32_t B = 0; B < k; B += 64) {
+                const uint32_t L = k - B < 64u ? k - B : 64u;
+                f += 4ull * L * chunk_groups(n, B, L);
+            }
+            widest = max(widest, n);
+        }
+        size[c] = f < 0x80000000ull ? (uint32_t)f : 0x80000000u;
+        sum += f;
+    }
+    part[threadIdx.x] = sum;
+    most[threadIdx.x] = widest;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) {
+            part[threadIdx.x] += part[threadIdx.x + w];
+            most[threadIdx.x] = max(most[threadIdx.x], most[threadIdx.x + w]);
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0 && part[0]) {
+        atomicAdd(&totals[0], part[0]);
+        atomicMax(&totals[1], (unsigned long long)most[0]);
+    }
+    if (blockIdx.x == 0) {
+        uint32_t pair = 0;
+        for (uint32_t z = threadIdx.x; z + 1 < a.nz; z += blockDim.x)
+            pair = max(pair, slice_pair(a, z, n_all).count);
+        atomicMax(&totals[2], (unsigned long long)pair);
+    }
+}
+
+// What a lane does at a step of the chain: exchange with the fraction (|f|
+// <= 0.5, or NaN), adopt the incoming value as its here-vorton (kAdopt: an
+// exchange at f = 1 from Omega_h = 0 gives Omega_h = Omega_t exactly), or
+// nothing (kSkip).
+constexpr float kAdopt = 1.0f, kSkip = -1.0f;
+
+// The fractions of every cell in the order of the chain's steps, one wave
+// per leaf point's cell: chunk by chunk, four steps of lane 0, of lane 1, ...
+// The same operations as the in-chain exchange, so the same bits.
 __global__ __launch_bounds__(256) void k_pse_fractions(PseArgs a, uint32_t cells,
+                                                       const float *__restrict__ alive,
+                                                       const uint32_t *__restrict__ frac_off,
                                                        float *__restrict__ frac) {
 #pragma clang fp contract(off)
     const uint32_t c = blockIdx.x * 4 + (threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63;
     if (c >= cells) return;
     const uint32_t k = a.count[c];
-    if (k < kSystolicMin) return;
-    const uint32_t nx = a.nx, nxy = a.nx * a.ny;
-    const uint32_t offs[8] = {0, 1, nx, 1 + nx, nxy, 1 + nxy, nx + nxy, 1 + nx + nxy};
-    uint32_t base[8], pre[9];
-    pre[0] = 0;
+    if (k == 0) return;
+    const CellPartners cp = cell_partners(a, c);
+    const uint32_t n = cp.pre[8];
+    float *__restrict__ fc = frac + frac_off[c];
+    for (uint32_t B = 0; B < k; B += 64) {
+        const uint32_t L = k - B < 64u ? k - B : 64u;
+        const uint32_t total = 4 * L * chunk_groups(n, B, L);
+        for (uint32_t q = lane; q < total; q += 64) {
+            const uint32_t g = q / (4 * L), r = q - g * (4 * L);
+            const uint32_t l = r >> 2, t = 4 * g + (r & 3u);
+            const uint32_t i = B + l, j = B + t - l;
+            float f = kSkip;
+            if (t >= l && j < n) {
+                if (j == i) {
+                    f = kAdopt;
+                } else if (j > i && alive[cp.base[0] + i] != 0.f) {
+                    const float4 ph = a.p[cp.base[0] + i];
+                    const float range = 4.0f * ph.w;
+                    f = pse_fraction(ph, range * range, a.p[partner_index(cp.base, cp.pre, j)],
+                                     a.nu_dt2);
+                }
+            }
+            fc[q] = f;
+        }
+        fc += total;
+    }
+}
+
+// Groups of four steps whose fractions a lane holds ahead of their use
+// (4, 6 and 8 groups: 3.88, 3.90 and 4.00 ms for the call at 1M vortons).
+constexpr int kRing = 4;
+
+// A cell as the chain takes it: its partners and its fractions.
+struct ChainCell {
+    CellPartners cp;
+    const float4 *F;
+};
+// What it is made of, one load for the wave: lanes 0-7 hold the cell's and
+// its forward cells' starts, lanes 8-15 their counts, the others the offset
+// of its fractions.  (Loaded one by one, each value waited for the one
+// before it and for the fractions in flight.)
+__device__ __forceinline__ uint32_t chain_cell_load(const PseArgs &a, uint32_t c,
+                                                    const uint32_t *__restrict__ frac_off,
+                                                    uint32_t lane) {
+    const uint32_t at = c + (lane & 1u) + ((lane & 2u) ? a.nx : 0u) +
+                        ((lane & 4u) ? a.nx * a.ny : 0u);
+    const uint32_t *src = lane < 8u ? a.start + at : lane < 16u ? a.count + at : frac_off + c;
+    return *src;
+}
+__device__ __forceinline__ ChainCell chain_cell(uint32_t v, const float *__restrict__ frac) {
+    ChainCell cell;
+    cell.cp.pre[0] = 0;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-        base[r] = a.start[c + offs[r]];
-        pre[r + 1] = pre[r] + a.count[c + offs[r]];
+        cell.cp.base[r] = (uint32_t)__builtin_amdgcn_readlane((int)v, r);
+        cell.cp.pre[r + 1] = cell.cp.pre[r] + (uint32_t)__builtin_amdgcn_readlane((int)v, 8 + r);
     }
-    const uint32_t n = pre[8];
-    float *__restrict__ fc = frac + a.frac_off[c];
-    const uint32_t total = k * n;
-    for (uint32_t q = lane; q < total; q += 64) {
-        const uint32_t i = q / n, j = q - i * n;
-        float f = 0.f;
-        if (j > i) {
-            const float4 ph = a.p[base[0] + i];
-            const float range = 4.0f * ph.w;
-            f = pse_fraction(ph, range * range, a.p[partner_index(base, pre, j)], a.nu_dt2);
-        }
-        fc[q] = f;
-    }
+    cell.F = reinterpret_cast<const float4 *>(
+        frac + (uint32_t)__builtin_amdgcn_readlane((int)v, 16));
+    return cell;
+}
+
+// What a lane holds of a chunk before its first step: whether its
+// here-vorton is alive, and the fractions of the first kRing groups.
+struct ChainLead {
+    float live;
+    float4 q[kRing];
+};
+__device__ __forceinline__ void lead_load(ChainLead &lead, const ChainCell &cell, const float4 *F,
+                                          uint32_t B, const float *__restrict__ alive,
+                                          uint32_t lane) {
+    const uint32_t k = cell.cp.pre[1], L = k - B < 64u ? k - B : 64u;
+    const uint32_t last = chunk_groups(cell.cp.pre[8], B, L) - 1, ll = lane < L ? lane : L - 1;
+    lead.live = alive[cell.cp.base[0] + B + ll];
+#pragma unroll
+    for (uint32_t r = 0; r < kRing; ++r) lead.q[r] = F[min(r, last) * L + ll];
+}
+
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// One component of Omega of one cell, by one wave: the systolic form (see
+// pse_cell_systolic) with the fractions precomputed.  The partners' values
+// wait in LDS (buf[0, n), filled by the caller); partner j of a chunk
+// starting at B enters lane 0 at step j - B, moves up one lane per step, and
+// leaves lane L - 1 back into buf, where the next chunk, or the write-back at
+// the end, finds it.  lead is the first chunk's; w is where the vortons'
+// values live, by index in the cell-sorted order.
+// The loops run at least once and load on every path, so that the compiler
+// can count the loads in flight and wait for the one it needs: with loads
+// behind a branch every group waited for the newest of them (5.4 against 3.1
+// ms for the two phases at 1M vortons).
+__device__ __forceinline__ void pse_cell_chain(const PseArgs &a, const ChainCell &cell,
+                                               ChainLead &lead,
+                                               const float *__restrict__ alive, float *w,
+                                               float *buf) {
+#pragma clang fp contract(off)
+    const uint32_t lane = threadIdx.x & 63;
+    const CellPartners &cp = cell.cp;
+    const uint32_t k = cp.pre[1], n = cp.pre[8];
+    const float4 *F = cell.F;
+    float4 (&q)[kRing] = lead.q;
+    uint32_t B = 0;
+    do {
+        const uint32_t L = k - B < 64u ? k - B : 64u;
+        const uint32_t groups = chunk_groups(n, B, L);
+        // lanes past the last follow it (they receive what leaves it)
+        const uint32_t ll = lane < L ? lane : L - 1;
+        const bool leaves = lane == L - 1;
+        float wh = 0.f, sw = 0.f;
+        float4 in = *reinterpret_cast<const float4 *>(buf + B);
+        float *out = buf + B - (L - 1);  // of the value leaving at step 0
+        uint32_t g0 = 0;
+        do {
+#pragma unroll
+            for (uint32_t r = 0; r < kRing; ++r) {
+                const uint32_t g = g0 + r;
+                if (g < groups) {
+                    const float f[4] = {q[r].x, q[r].y, q[r].z, q[r].w};
+                    const float v[4] = {in.x, in.y, in.z, in.w};
+                    in = *reinterpret_cast<const float4 *>(buf + B + 4 * (g + 1));
+                    float o[4];
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        sw = wave_shr(sw, v[d]);  // lane 0 takes the next partner
+                        const float e = (wh - sw) * f[d];
+                        const float ex = f[d] != kSkip ? e : 0.f;
+                        wh -= ex;
+                        sw += ex;
+                        o[d] = sw;
+                    }
+                    // values below B belong to steps before the first partner
+                    // has passed; their places in buf are no longer read
+                    if (4 * g + 3 >= L - 1 && leaves) {
+#pragma unroll
+                        for (int d = 0; d < 4; ++d) out[4 * g + d] = o[d];
+                    }
+                }
+                q[r] = F[min(g + kRing, groups - 1) * L + ll];
+            }
+            g0 += kRing;
+        } while (g0 < groups);
+        F += groups * L;
+        if (lead.live != 0.f) wh -= wh * a.dissipation;
+        if (lane < L) w[cp.base[0] + B + lane] = wh;
+        B += 64;
+        if (B < k) lead_load(lead, cell, F, B, alive, lane);
+    } while (B < k);
+    wave_lds_fence();
+    for (uint32_t j = k + lane; j < n; j += 64) w[partner_index(cp.base, cp.pre, j)] = buf[j];
 }
 
 // Cells of wavefront step t of a slice: x + 2y = t, y from
@@ -504,17 +610,16 @@ __device__ __forceinline__ void step_rows(int t, int cx, int cy, int &ylo, int &
 
 // Work of a cell in steps of pse_cell_wave: the partner stream of each chunk
 // of 64 here-vortons in the systolic form, k n in the small-cell form; 0 for
-// an empty cell (nothing to do), at least 1 otherwise.
+// an empty cell (nothing to do), at least 1 otherwise.  The chain form
+// (CHAIN) is systolic throughout and pays about 24 steps' time per cell for
+// its loads and stores.
+template <bool CHAIN>
 __device__ __forceinline__ uint32_t cell_cost(const PseArgs &a, uint32_t c) {
-    const uint32_t nx = a.nx, nxy = a.nx * a.ny;
     const uint32_t k = a.count[c];
     if (k == 0) return 0u;
-    const uint32_t offs[8] = {0, 1, nx, 1 + nx, nxy, 1 + nxy, nx + nxy, 1 + nx + nxy};
-    uint32_t n = 0;
-#pragma unroll
-    for (int r = 0; r < 8; ++r) n += a.count[c + offs[r]];
-    uint64_t cost = 0;
-    if (k < kSystolicMin) {
+    const uint32_t n = cell_partners(a, c).pre[8];
+    uint64_t cost = CHAIN ? 24 : 0;
+    if (!CHAIN && k < kSystolicMin) {
         cost = (uint64_t)k * n;
     } else {
         for (uint32_t b = 0; b < k; b += 64) cost += (n - b) + (k - b < 64u ? k - b : 64u) - 1;
@@ -528,10 +633,11 @@ __device__ __forceinline__ uint32_t cell_cost(const PseArgs &a, uint32_t c) {
 // wave.  One wave per (step t, slice z) assigns the step's non-empty cells,
 // largest first, each to the wave with the least work so far (greedy LPT),
 // and writes them grouped by wave: perm[sched * M + i] for i in
-// [wstart[9 sched + w], wstart[9 sched + w + 1]), sched = z steps + t.
-// Up to kSchedSlots * 64 cells per step.
+// [wstart[(WAVES + 1) sched + w], wstart[(WAVES + 1) sched + w + 1]), sched =
+// z steps + t.  Up to kSchedSlots * 64 cells per step.
 constexpr int kSchedSlots = 4;
 
+template <int WAVES, bool CHAIN>
 __global__ __launch_bounds__(64) void k_pse_schedule(PseArgs a, uint32_t steps, uint32_t M,
                                                      uint32_t *__restrict__ perm,
                                                      uint32_t *__restrict__ wstart) {
@@ -547,13 +653,13 @@ __global__ __launch_bounds__(64) void k_pse_schedule(PseArgs a, uint32_t steps, 
 #pragma unroll
     for (int q = 0; q < kSchedSlots; ++q) {
         const int y = ylo + lane + 64 * q;
-        rem[q] = y <= yhi ? cell_cost(a, (uint32_t)(t - 2 * y) + nx * (uint32_t)y + nxy * z) : 0u;
+        rem[q] = y <= yhi ? cell_cost<CHAIN>(a, (uint32_t)(t - 2 * y) + nx * (uint32_t)y + nxy * z) : 0u;
         slot_w[q] = -1;
         slot_pos[q] = 0;
     }
-    uint32_t load[kPseWaves], cnt[kPseWaves];
+    uint32_t load[WAVES], cnt[WAVES];
 #pragma unroll
-    for (int w = 0; w < kPseWaves; ++w) load[w] = cnt[w] = 0u;
+    for (int w = 0; w < WAVES; ++w) load[w] = cnt[w] = 0u;
     for (;;) {
         uint32_t best = rem[0];
 #pragma unroll
@@ -577,10 +683,10 @@ __global__ __launch_bounds__(64) void k_pse_schedule(PseArgs a, uint32_t steps, 
         }
         int w = 0;
 #pragma unroll
-        for (int v = 1; v < kPseWaves; ++v) w = load[v] < load[w] ? v : w;
+        for (int v = 1; v < WAVES; ++v) w = load[v] < load[w] ? v : w;
         uint32_t pos = 0;
 #pragma unroll
-        for (int v = 0; v < kPseWaves; ++v) {
+        for (int v = 0; v < WAVES; ++v) {
             if (v == w) {
                 pos = cnt[v];
                 cnt[v] += 1u;
@@ -596,26 +702,163 @@ __global__ __launch_bounds__(64) void k_pse_schedule(PseArgs a, uint32_t steps, 
             }
         }
     }
-    uint32_t ws[kPseWaves + 1];
+    uint32_t ws[WAVES + 1];
     ws[0] = 0;
 #pragma unroll
-    for (int v = 0; v < kPseWaves; ++v) ws[v + 1] = ws[v] + cnt[v];
+    for (int v = 0; v < WAVES; ++v) ws[v + 1] = ws[v] + cnt[v];
     const size_t sched = (size_t)z * steps + (size_t)t;
-    if (lane <= kPseWaves) {
+    if (lane <= WAVES) {
         uint32_t v = 0;
 #pragma unroll
-        for (int u = 0; u <= kPseWaves; ++u) v = lane == u ? ws[u] : v;
-        wstart[(kPseWaves + 1) * sched + (size_t)lane] = v;
+        for (int u = 0; u <= WAVES; ++u) v = lane == u ? ws[u] : v;
+        wstart[(WAVES + 1) * sched + (size_t)lane] = v;
     }
 #pragma unroll
     for (int q = 0; q < kSchedSlots; ++q) {
         if (slot_w[q] >= 0) {
             uint32_t base = 0;
 #pragma unroll
-            for (int u = 0; u < kPseWaves; ++u) base = slot_w[q] == u ? ws[u] : base;
+            for (int u = 0; u < WAVES; ++u) base = slot_w[q] == u ? ws[u] : base;
             perm[sched * M + base + (uint32_t)slot_pos[q]] = (uint32_t)(ylo + lane + 64 * q);
         }
     }
+}
+
+// The schedule as one list per slice and wave: cells (step << 16 | y) in step
+// order, list[z steps M + lstart[(kChainWaves + 1) z + w] ...].
+__global__ __launch_bounds__(kChainThreads) void k_pse_lists(uint32_t steps, uint32_t M,
+                                                             const uint32_t *__restrict__ perm,
+                                                             const uint32_t *__restrict__ wstart,
+                                                             uint32_t *__restrict__ list,
+                                                             uint32_t *__restrict__ lstart) {
+    __shared__ uint32_t total[kChainWaves];
+    const uint32_t z = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    auto cells = [&](uint32_t t, uint32_t &b, uint32_t &e) {
+        const size_t at = (kChainWaves + 1) * ((size_t)z * steps + t) + wave;
+        b = wstart[at];
+        e = wstart[at + 1];
+    };
+    uint32_t sum = 0, b, e;
+    for (uint32_t t = lane; t < steps; t += 64) {
+        cells(t, b, e);
+        sum += e - b;
+    }
+    for (int off = 32; off > 0; off >>= 1) sum += (uint32_t)__shfl_xor((int)sum, off, 64);
+    if (lane == 0) total[wave] = sum;
+    __syncthreads();
+    uint32_t at = 0;
+    for (uint32_t v = 0; v < wave; ++v) at += total[v];
+    if (lane == 0) {
+        lstart[(kChainWaves + 1) * z + wave] = at;
+        if (wave + 1 == kChainWaves) lstart[(kChainWaves + 1) * z + kChainWaves] = at + sum;
+    }
+    const size_t region = (size_t)z * steps * M;
+    for (uint32_t t0 = 0; t0 < steps; t0 += 64) {
+        const uint32_t t = t0 + lane;
+        b = e = 0;
+        if (t < steps) cells(t, b, e);
+        uint32_t incl = e - b;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = (uint32_t)__shfl_up((int)incl, off, 64);
+            if ((int)lane >= off) incl += o;
+        }
+        uint32_t p = at + incl - (e - b);
+        for (uint32_t i = b; i < e; ++i)
+            list[region + p++] = (t << 16) | perm[((size_t)z * steps + t) * M + i];
+        at += (uint32_t)__shfl((int)incl, 63, 64);
+    }
+}
+
+// One component (blockIdx.y) of one slice z = phase + 2 blockIdx.x: every wave
+// goes through its list of cells, with a workgroup barrier between wavefront
+// steps.  What a cell needs besides Omega does not change during the call,
+// so the next cell's partners and first fractions are fetched while the
+// current one runs.
+// RESIDENT: the component of both slices' vortons stays in LDS for the whole
+// phase (`buf_floats` per wave, then the values), so a step waits for no
+// global load or store: 3.88 against 4.10 ms for the call at 1M vortons.
+// Otherwise (slices too full for the LDS) they stay in w3.
+template <bool RESIDENT>
+__global__ __launch_bounds__(kChainThreads) void k_pse_phase_chain(
+    PseArgs a, uint32_t phase, uint32_t steps, uint32_t M, const uint32_t *__restrict__ list,
+    const uint32_t *__restrict__ lstart, const float *__restrict__ frac,
+    const uint32_t *__restrict__ frac_off, const float *__restrict__ alive, float *w3, uint32_t n,
+    uint32_t buf_floats) {
+    extern __shared__ __align__(16) float lds[];
+    const uint32_t z = phase + 2 * blockIdx.x;
+    if (z + 1 >= a.nz) return;  // uniform per workgroup
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float *global = w3 + (size_t)blockIdx.y * n;
+    float *buf = lds + wave * buf_floats + kBufFront;
+    const SlicePair pair = slice_pair(a, z, n);
+    float *resident = lds + kChainWaves * buf_floats;
+    float *w = RESIDENT ? resident - pair.first : global;
+    if (RESIDENT) {
+        for (uint32_t i = threadIdx.x; i < pair.count; i += kChainThreads)
+            resident[i] = global[pair.first + i];
+        __syncthreads();
+    }
+    auto next_step = [&] {
+        // LDS is all that the waves share: nothing waits for the fractions
+        // in flight
+        if (RESIDENT)
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else
+            __syncthreads();
+    };
+    const uint32_t *cells = list + (size_t)z * steps * M;
+    uint32_t p = __builtin_amdgcn_readfirstlane(lstart[(kChainWaves + 1) * z + wave]);
+    const uint32_t end =
+        __builtin_amdgcn_readfirstlane(lstart[(kChainWaves + 1) * z + wave + 1]);
+    // the list's last cell stands in for those after it
+    auto entry_at = [&](uint32_t i) {
+        return __builtin_amdgcn_readfirstlane(cells[min(i, end - 1)]);
+    };
+    auto load = [&](uint32_t entry) {
+        const uint32_t t = entry >> 16, y = entry & 0xffffu;
+        return chain_cell_load(a, (t - 2 * y) + a.nx * (y + a.ny * z), frac_off, lane);
+    };
+    uint32_t now = 0;  // barriers passed: the current wavefront step
+    if (p < end) {
+        uint32_t entry = entry_at(p), entry1 = entry_at(p + 1), entry2 = cells[min(p + 2, end - 1)];
+        ChainCell cell = chain_cell(load(entry), frac);
+        uint32_t v1 = load(entry1);
+        ChainLead lead, lead1;
+        lead_load(lead, cell, cell.F, 0, alive, lane);
+        for (; p < end; ++p) {
+            const ChainCell cell1 = chain_cell(v1, frac);
+            const uint32_t e2 = __builtin_amdgcn_readfirstlane(entry2);
+            v1 = load(e2);
+            entry2 = cells[min(p + 3, end - 1)];
+            lead_load(lead1, cell1, cell1.F, 0, alive, lane);
+            for (; now < (entry >> 16); ++now) next_step();
+            const uint32_t np = cell.cp.pre[8];
+            for (uint32_t j0 = 0; j0 < np; j0 += 256) {
+                float v[4];
+#pragma unroll
+                for (uint32_t r = 0; r < 4; ++r) {
+                    const uint32_t j = j0 + 64 * r + lane;
+                    if (j < np) v[r] = w[partner_index(cell.cp.base, cell.cp.pre, j)];
+                }
+#pragma unroll
+                for (uint32_t r = 0; r < 4; ++r) {
+                    const uint32_t j = j0 + 64 * r + lane;
+                    if (j < np) buf[j] = v[r];
+                }
+            }
+            wave_lds_fence();
+            pse_cell_chain(a, cell, lead, alive, w, buf);
+            lead = lead1;
+            cell = cell1;
+            entry = entry1;
+            entry1 = e2;
+        }
+    }
+    for (; now < steps; ++now) next_step();
+    if (RESIDENT)
+        for (uint32_t i = threadIdx.x; i < pair.count; i += kChainThreads)
+            global[pair.first + i] = resident[i];
 }
 
 // perm / wstart: the schedule of k_pse_schedule, or null for round robin by
@@ -760,6 +1003,31 @@ __global__ void k_pse_scatter(const uint32_t *__restrict__ idx, const float4 *__
     o[2] = v.z;
 }
 
+// One array per component, and which vortons are alive.
+__global__ void k_pse_gather3(const uint32_t *__restrict__ idx, const float *__restrict__ angvel,
+                              size_t ang_stride, const int32_t *__restrict__ birth,
+                              size_t birth_stride, size_t n, float *__restrict__ w3,
+                              float *__restrict__ alive) {
+    const size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= n) return;
+    const size_t i = idx[j];
+    const float *o = angvel + i * ang_stride;
+    w3[j] = o[0];
+    w3[n + j] = o[1];
+    w3[2 * n + j] = o[2];
+    alive[j] = !birth || birth[i * birth_stride] >= 0 ? 1.f : 0.f;
+}
+
+__global__ void k_pse_scatter3(const uint32_t *__restrict__ idx, const float *__restrict__ w3,
+                               size_t n, float *__restrict__ angvel, size_t ang_stride) {
+    const size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= n) return;
+    float *o = angvel + (size_t)idx[j] * ang_stride;
+    o[0] = w3[j];
+    o[1] = w3[n + j];
+    o[2] = w3[2 * n + j];
+}
+
 }  // namespace
 
 vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const int32_t *birth,
@@ -785,89 +1053,130 @@ vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const 
     a.w = w;
     a.nu_dt2 = 2.0f * viscosity * dt;   // 2.0f * mViscosity * timeStep
     a.dissipation = viscosity * dt;     // mViscosity * timeStep
-    a.frac = nullptr;
-    a.frac_off = nullptr;
-    vg_status st = launch("vg_pse_gather", k_pse_gather, dim3(ceil_div(n, 256)), dim3(256), 0, s,
-                          tv.sorted_idx, (const float *)angvel, ang_stride, birth, birth_stride,
-                          n, w);
-    const float4 *result = w;
     if (sim) {
+        vg_status st = launch("vg_pse_gather", k_pse_gather, dim3(ceil_div(n, 256)), dim3(256), 0,
+                              s, tv.sorted_idx, (const float *)angvel, ang_stride, birth,
+                              birth_stride, n, w);
         if (st == VG_OK)
             st = launch("vg_pse_simultaneous", k_pse_simultaneous, dim3(ceil_div(n, 256)),
                         dim3(256), 0, s, a, g, (const float4 *)w, w + n, (uint32_t)n);
-        result = w + n;
-    } else {
-        const uint32_t slices = a.nz - 1;  // cell slices 0 .. nz-2
-        const uint32_t cx = a.nx - 1, cy = a.ny - 1;
-        const uint32_t steps = (cx - 1) + 2 * (cy - 1) + 1;
-        // cells per wavefront step are at most min(cy, (cx + 1) / 2)
-        const uint32_t M = cy < (cx + 1) / 2 ? cy : (cx + 1) / 2;
-        uint32_t *perm = nullptr, *wstart = nullptr;
-        const size_t nsched = (size_t)slices * steps;
-        // exchange fractions of the systolic cells, computed over the whole
-        // chip before the serial phases (the block sizes are read back to
-        // size the buffer: one stream synchronisation)
-        const size_t cells = capacity(g);
-        uint32_t *fsize = nullptr, *foff = nullptr, *stmp = nullptr;
-        unsigned long long *dtot = nullptr;
-        float *frac = nullptr;
-        if (st == VG_OK) st = salloc((void **)&fsize, cells * sizeof(uint32_t), s);
-        if (st == VG_OK) st = salloc((void **)&foff, cells * sizeof(uint32_t), s);
-        if (st == VG_OK) st = salloc((void **)&stmp, scan_scratch_elems(cells) * sizeof(uint32_t), s);
-        if (st == VG_OK) st = salloc((void **)&dtot, sizeof(unsigned long long), s);
-        if (st == VG_OK) st = launch("vg_pse_frac_size", k_pse_zero64, dim3(1), dim3(1), 0, s, dtot);
         if (st == VG_OK)
-            st = launch("vg_pse_frac_size", k_pse_frac_size, dim3(ceil_div(cells, 256)), dim3(256),
-                        0, s, a, (uint32_t)cells, fsize, dtot);
-        if (st == VG_OK) st = exclusive_scan_u32(fsize, foff, cells, stmp, s);
-        unsigned long long total = 0;
+            st = launch("vg_pse_scatter", k_pse_scatter, dim3(ceil_div(n, 256)), dim3(256), 0, s,
+                        tv.sorted_idx, (const float4 *)(w + n), n, angvel, ang_stride);
+        sfree(w, s);
+        return st;
+    }
+    const uint32_t slices = a.nz - 1;  // cell slices 0 .. nz-2
+    const uint32_t cx = a.nx - 1, cy = a.ny - 1;
+    const uint32_t steps = (cx - 1) + 2 * (cy - 1) + 1;
+    // cells per wavefront step are at most min(cy, (cx + 1) / 2)
+    const uint32_t M = cy < (cx + 1) / 2 ? cy : (cx + 1) / 2;
+    const size_t nsched = (size_t)slices * steps, cells = capacity(g);
+    uint32_t *perm = nullptr, *wstart = nullptr, *fsize = nullptr, *foff = nullptr,
+             *stmp = nullptr, *list = nullptr, *lstart = nullptr;
+    unsigned long long *dtot = nullptr;
+    float *frac = nullptr;
+    // The fractions' sizes are read back to size their buffer: one stream
+    // synchronisation.
+    vg_status st = salloc((void **)&fsize, cells * sizeof(uint32_t), s);
+    if (st == VG_OK) st = salloc((void **)&foff, cells * sizeof(uint32_t), s);
+    if (st == VG_OK) st = salloc((void **)&stmp, scan_scratch_elems(cells) * sizeof(uint32_t), s);
+    if (st == VG_OK) st = salloc((void **)&dtot, 3 * sizeof(unsigned long long), s);
+    if (st == VG_OK) st = launch("vg_pse_frac_size", k_pse_zero64, dim3(1), dim3(3), 0, s, dtot);
+    if (st == VG_OK)
+        st = launch("vg_pse_frac_size", k_pse_frac_size,
+                    dim3(min(ceil_div(cells, 256), 1024u)), dim3(256), 0, s, a, (uint32_t)cells,
+                    (uint32_t)n, fsize, dtot);
+    if (st == VG_OK) st = exclusive_scan_u32(fsize, foff, cells, stmp, s);
+    unsigned long long totals[3] = {0, 0, 0};
+    if (st == VG_OK) {
+        hipError_t e = hipMemcpyAsync(totals, dtot, sizeof totals, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e != hipSuccess) {
+            set_error(std::string("PSE fraction sizes: ") + hipGetErrorString(e));
+            st = VG_EDEVICE;
+        }
+    }
+    // Fractions of 2^31 floats or more, and cells whose partners do not fit
+    // a wave's LDS, keep the fractions in the chain, and so does
+    // VG_PSE_FRACTIONS=0 in the environment (the same bits either way; the
+    // switch keeps that path testable).
+    const char *env = getenv("VG_PSE_FRACTIONS");
+    const bool scheduled = M <= 64u * kSchedSlots && nsched * M < (size_t(1) << 28);
+    const bool chain = !(env && env[0] == '0') && totals[0] > 0 && totals[0] < (1ull << 31) &&
+                       totals[1] <= kChainPartners && scheduled && steps < (1u << 16);
+    const uint32_t waves = chain ? kChainWaves : kPseWaves;
+    if (st == VG_OK && scheduled) {
+        st = salloc((void **)&perm, nsched * M * sizeof(uint32_t), s);
+        if (st == VG_OK) st = salloc((void **)&wstart, nsched * (waves + 1) * sizeof(uint32_t), s);
+        if (st == VG_OK)
+            st = launch("vg_pse_schedule",
+                        chain ? k_pse_schedule<kChainWaves, true> : k_pse_schedule<kPseWaves, false>,
+                        dim3(steps, slices), dim3(64), 0, s, a, steps, M, perm, wstart);
+    }
+    if (chain) {
+        float *w3 = reinterpret_cast<float *>(w), *alive = w3 + 3 * n;
+        if (st == VG_OK) st = salloc((void **)&list, nsched * M * sizeof(uint32_t), s);
+        if (st == VG_OK)
+            st = salloc((void **)&lstart, slices * (kChainWaves + 1) * sizeof(uint32_t), s);
+        if (st == VG_OK)
+            st = launch("vg_pse_schedule", k_pse_lists, dim3(slices), dim3(kChainThreads), 0, s,
+                        steps, M, (const uint32_t *)perm, (const uint32_t *)wstart, list, lstart);
+        if (st == VG_OK) st = salloc((void **)&frac, totals[0] * sizeof(float), s);
+        if (st == VG_OK)
+            st = launch("vg_pse_gather", k_pse_gather3, dim3(ceil_div(n, 256)), dim3(256), 0, s,
+                        tv.sorted_idx, (const float *)angvel, ang_stride, birth, birth_stride, n,
+                        w3, alive);
+        if (st == VG_OK)
+            st = launch("vg_pse_fractions", k_pse_fractions,
+                        dim3(ceil_div(cells, 4)), dim3(256), 0, s, a, (uint32_t)cells, (const float *)alive, (const uint32_t *)foff,
+                        frac);
+        const uint32_t buf_floats = kBufFront + (((uint32_t)totals[1] + 3u) & ~3u) + kBufBack;
+        size_t lds = kChainWaves * buf_floats * sizeof(float);
+        const bool resident = lds + totals[2] * sizeof(float) <= kLdsBytes;
+        if (resident) lds += totals[2] * sizeof(float);
+        const auto kernel = resident ? k_pse_phase_chain<true> : k_pse_phase_chain<false>;
         if (st == VG_OK) {
-            hipError_t e = hipMemcpyAsync(&total, dtot, sizeof total, hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess) e = hipStreamSynchronize(s);
-            if (e != hipSuccess) {
-                set_error(std::string("PSE fraction sizes: ") + hipGetErrorString(e));
-                st = VG_EDEVICE;
-            }
-        }
-        // blocks of 2^31 floats or more keep the in-chain fractions, and so
-        // does VG_PSE_FRACTIONS=0 in the environment (the same bits either
-        // way; the switch keeps the in-chain path testable)
-        const char *env = getenv("VG_PSE_FRACTIONS");
-        const bool precompute = !(env && env[0] == '0');
-        if (st == VG_OK && precompute && total > 0 && total < (1ull << 31)) {
-            st = salloc((void **)&frac, total * sizeof(float), s);
-            if (st == VG_OK) {
-                a.frac = frac;
-                a.frac_off = foff;
-                st = launch("vg_pse_fractions", k_pse_fractions, dim3(ceil_div(cells, 4)),
-                            dim3(256), 0, s, a, (uint32_t)cells, frac);
-            }
-        }
-        if (st == VG_OK && M <= 64u * kSchedSlots && nsched * M < (size_t(1) << 28)) {
-            st = salloc((void **)&perm, nsched * M * sizeof(uint32_t), s);
-            if (st == VG_OK)
-                st = salloc((void **)&wstart, nsched * (kPseWaves + 1) * sizeof(uint32_t), s);
-            if (st == VG_OK)
-                st = launch("vg_pse_schedule", k_pse_schedule, dim3(steps, slices), dim3(64), 0, s,
-                            a, steps, M, perm, wstart);
+            const hipError_t e =
+                hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
+            if (e != hipSuccess) st = device_error(e, "PSE LDS size", __FILE__, __LINE__);
         }
         for (uint32_t phase = 0; phase < 2 && st == VG_OK; ++phase) {
             const uint32_t groups = (slices - phase + 1) / 2;
             if (groups)
-                st = launch("vg_pse_phase", k_pse_phase, dim3(groups), dim3(kPseThreads), 0, s,
-                            a, phase, (const uint32_t *)perm, (const uint32_t *)wstart, M);
+                st = launch("vg_pse_phase", kernel, dim3(groups, 3), dim3(kChainThreads), lds, s,
+                            a, phase, steps, M, (const uint32_t *)list, (const uint32_t *)lstart,
+                            (const float *)frac, (const uint32_t *)foff, (const float *)alive, w3,
+                            (uint32_t)n, buf_floats);
         }
-        if (perm) sfree(perm, s);
-        if (wstart) sfree(wstart, s);
-        if (frac) sfree(frac, s);
-        if (fsize) sfree(fsize, s);
-        if (foff) sfree(foff, s);
-        if (stmp) sfree(stmp, s);
-        if (dtot) sfree(dtot, s);
+        if (st == VG_OK)
+            st = launch("vg_pse_scatter", k_pse_scatter3, dim3(ceil_div(n, 256)), dim3(256), 0, s,
+                        tv.sorted_idx, (const float *)w3, n, angvel, ang_stride);
+    } else {
+        if (st == VG_OK)
+            st = launch("vg_pse_gather", k_pse_gather, dim3(ceil_div(n, 256)), dim3(256), 0, s,
+                        tv.sorted_idx, (const float *)angvel, ang_stride, birth, birth_stride, n,
+                        w);
+        for (uint32_t phase = 0; phase < 2 && st == VG_OK; ++phase) {
+            const uint32_t groups = (slices - phase + 1) / 2;
+            if (groups)
+                st = launch("vg_pse_phase", k_pse_phase, dim3(groups), dim3(kPseThreads), 0, s, a,
+                            phase, (const uint32_t *)perm, (const uint32_t *)wstart, M);
+        }
+        if (st == VG_OK)
+            st = launch("vg_pse_scatter", k_pse_scatter, dim3(ceil_div(n, 256)), dim3(256), 0, s,
+                        tv.sorted_idx, (const float4 *)w, n, angvel, ang_stride);
     }
-    if (st == VG_OK)
-        st = launch("vg_pse_scatter", k_pse_scatter, dim3(ceil_div(n, 256)), dim3(256), 0, s,
-                    tv.sorted_idx, result, n, angvel, ang_stride);
+    if (perm) sfree(perm, s);
+    if (wstart) sfree(wstart, s);
+    if (list) sfree(list, s);
+    if (lstart) sfree(lstart, s);
+    if (frac) sfree(frac, s);
+    if (fsize) sfree(fsize, s);
+    if (foff) sfree(foff, s);
+    if (stmp) sfree(stmp, s);
+    if (dtot) sfree(dtot, s);
     sfree(w, s);
     return st;
 }
