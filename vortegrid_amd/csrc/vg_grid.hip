@@ -8,7 +8,10 @@
 // All stencil arithmetic here is HBM/MALL bound and compiled with FP
 // contraction off, so results match the reference's operation order bit for
 // bit.
+#include <algorithm>
+#include <cmath>
 #include <cstring>
+#include <utility>
 #include <vector>
 
 #include "vg_internal.h"
@@ -196,6 +199,196 @@ __global__ __launch_bounds__(64) void k_sor_rows_split(vg_grid_desc g, float *__
             l = nv;
             cur = xp[u];
         }
+    }
+}
+
+// Several colour passes of one component in LDS.
+//
+// A colour pass has little work and a long serial chain (x in place), so the
+// row kernels above spend it waiting: for their inputs' round trips to L2,
+// and, on small grids, for the launch.  Here a workgroup stages whole x rows
+// of a block of (y, z) rows and `passes` rows around it, and runs that many
+// passes on them: rows of one colour read only rows of the other, so after p
+// passes every staged row at least p rows away from the staged edge holds
+// the value the whole grid's pass would give it, by the same operations
+// (bit for bit).  The owned rows go out; the rows around them, which
+// neighbouring workgroups own, are recomputed rather than exchanged.  A grid
+// whose component fits one workgroup's LDS runs all its passes in one launch
+// with nothing around it.
+//
+// The passes follow each other down the rows: a row is swept in chunks of
+// kSorChunk points, and pass p sweeps chunk c at tick p + c, one barrier per
+// tick.  Its chunk reads the other colour's rows in that chunk, which pass
+// p - 1 swept a tick earlier, and of its own rows the first point of the next
+// chunk, which pass p - 2 did; pass p - 1, at the next chunk, reads nothing
+// that pass p writes.  So `slots` passes are in flight, each on its own
+// waves, and the chain that a workgroup waits for is passes + chunks ticks
+// long instead of passes x chunks.
+//
+// Lanes take rows; rows lie nx floats apart, an odd number (every
+// power-of-two grid's; others keep the row kernels), so a wave's reads at one
+// x fall on different banks.  One step of a row takes about 20
+// instructions, 160 cycles for a wave alone on its SIMD.
+//
+// Per cascade visit of 32 passes, against one launch per pass: 65x65x129
+// 185 against 610 us, 33x33x65 97 against 250 us, 17x17x33 44 against 130
+// us, 9x9x17 and smaller 24 against 110 us; the 262,144-vorton POISSON update
+// 2.78 -> 1.07 ms.
+struct SorBlock {
+    int nx, ny, nz;
+    int by, bz;       // owned rows per workgroup
+    int passes;       // colour passes of this launch = rows staged around
+    int color;        // of the first pass
+    int slots;        // passes in flight
+    int slot_threads; // lanes (rows of one colour, or fewer) per slot
+    uint32_t in_mul, out_mul, f_mul;  // value (component k, point o) at o mul + k comp
+    size_t in_comp, out_comp, f_comp;
+};
+constexpr int kSorThreads = 1024, kSorChunk = 8, kSorStage = 16;
+constexpr size_t kSorLdsBytes = 160 * 1024;  // of a CU
+
+__global__ __launch_bounds__(kSorThreads) void k_sor_block(SorBlock b, const float *in, float *out,
+                                                           const float *__restrict__ lap,
+                                                           SorCoef c) {
+#pragma clang fp contract(off)
+    extern __shared__ float lds[];
+    const int tid = (int)threadIdx.x, nx = b.nx, ny = b.ny, nz = b.nz;
+    const int y0 = 1 + (int)blockIdx.x * b.by, z0 = 1 + (int)blockIdx.y * b.bz;
+    const int y1 = min(y0 + b.by, ny - 1), z1 = min(z0 + b.bz, nz - 1);
+    const int ya = max(0, y0 - b.passes), yb = min(ny, y1 + b.passes);
+    const int za = max(0, z0 - b.passes), zb = min(nz, z1 + b.passes);
+    const int ey = yb - ya, ez = zb - za;
+    float *u = lds, *fl = lds + ey * ez * nx;  // fl: the staged rows but the outermost
+    const size_t k = blockIdx.z;
+    in += k * b.in_comp;
+    out += k * b.out_comp;
+    lap += k * b.f_comp;
+    const int threads = (int)blockDim.x;
+    // Rows [ra, rb) x [sa, sb) of (y, z): one run of points per z, in LDS
+    // (row (y, z) = row y - la of ly in plane z - ma) as in memory, since the
+    // rows' stride is nx in both.  get(LDS index, point) of kSorStage points
+    // of a thread is under way before put(LDS index, point, value) takes the
+    // first.
+    auto runs = [&](int ra, int rb, int sa, int sb, int la, int ma, int ly, auto &&get,
+                    auto &&put) {
+        const int run = (rb - ra) * nx, total = run * (sb - sa);
+        const int skip_at = (ly - (rb - ra)) * nx, skip_o = (ny - (rb - ra)) * nx;
+        // point tid + j threads: `qt` runs and q1 points further each time
+        const int t = tid / run, qt = threads / run, q1 = threads - qt * run;
+        int i = tid - t * run;
+        int at = (ra - la + ly * (sa - ma)) * nx + tid + t * skip_at;
+        int o = (ra + ny * sa) * nx + tid + t * skip_o;
+        const int step_at = threads + qt * skip_at, step_o = threads + qt * skip_o;
+        for (int e = tid; e < total; e += kSorStage * threads) {
+            int ats[kSorStage], os[kSorStage];
+            float v[kSorStage];
+#pragma unroll
+            for (int j = 0; j < kSorStage; ++j) {
+                ats[j] = at;
+                os[j] = o;
+                if (e + j * threads < total) v[j] = get(at, (uint32_t)o);
+                i += q1;
+                const bool next = i >= run;
+                i -= next ? run : 0;
+                at += step_at + (next ? skip_at : 0);
+                o += step_o + (next ? skip_o : 0);
+            }
+#pragma unroll
+            for (int j = 0; j < kSorStage; ++j)
+                if (e + j * threads < total) put(ats[j], (uint32_t)os[j], v[j]);
+        }
+    };
+    runs(ya, yb, za, zb, ya, za, ey, [&](int, uint32_t o) { return in[o * b.in_mul]; },
+         [&](int at, uint32_t, float v) { u[at] = v; });
+    runs(ya + 1, yb - 1, za + 1, zb - 1, ya + 1, za + 1, ey - 2,
+         [&](int, uint32_t o) { return lap[o * b.f_mul]; },
+         [&](int at, uint32_t, float v) { fl[at] = v; });
+    __syncthreads();
+    // The row (y, z) r of a colour among the staged rows that have neighbours.
+    const int half = (ey - 1) / 2, rows = half * (ez - 2);
+    auto row_of = [&](int r, int color, int &y, int &z) {
+        const int q = r / half;
+        z = za + 1 + q;
+        y = ya + 1 + ((ya + 1 + z + color) & 1) + 2 * (r - q * half);
+    };
+    // a slot is whole waves, so its pass and chunk are a wave's
+    const int slot = __builtin_amdgcn_readfirstlane(tid / b.slot_threads);
+    const int r0 = tid - slot * b.slot_threads;
+    int y0c, z0c, y1c, z1c;  // row r0 of either colour
+    row_of(r0, 0, y0c, z0c);
+    row_of(r0, 1, y1c, z1c);
+    auto u_at = [&](int y, int z) { return ((y - ya) + ey * (z - za)) * nx; };
+    auto f_at = [&](int y, int z) { return ((y - ya - 1) + (ey - 2) * (z - za - 1)) * nx; };
+    const int u0 = u_at(y0c, z0c), u1 = u_at(y1c, z1c), f0 = f_at(y0c, z0c), f1 = f_at(y1c, z1c);
+    const int up = ey * nx;
+    const int chunks = (nx - 2 + kSorChunk - 1) / kSorChunk, period = max(chunks, b.slots);
+    const int ticks = (b.passes - 1) / b.slots * period + (b.passes - 1) % b.slots + chunks;
+    // One chunk of one row: points past the row's end read what lies behind
+    // it (the LDS has room for that) and are not swept.
+    auto sweep = [&](float *row, const float *fr, int left) {
+        float xp[kSorChunk], ys[kSorChunk], zs[kSorChunk], f[kSorChunk];
+        float l = row[-1], cur = row[0];
+#pragma unroll
+        for (int i = 0; i < kSorChunk; ++i) {
+            xp[i] = row[i + 1];
+            ys[i] = row[i + nx] + row[i - nx];
+            zs[i] = row[i + up] + row[i - up];
+            f[i] = fr[i];
+        }
+        auto step = [&](int i) {
+            const float a = ((xp[i] + l) * c.r2x + ys[i] * c.r2y + zs[i] * c.r2z - f[i]) * c.h;
+            l = c.omr * cur + c.relax * a;
+            row[i] = l;
+            cur = xp[i];
+        };
+        if (left >= kSorChunk) {
+#pragma unroll
+            for (int i = 0; i < kSorChunk; ++i) step(i);
+        } else {
+#pragma unroll
+            for (int i = 0; i < kSorChunk - 1; ++i)
+                if (i < left) step(i);
+        }
+    };
+    int p = slot, chunk = -slot;  // of this slot at the current tick
+    for (int t = 0; t < ticks; ++t) {
+        if (slot < b.slots && chunk >= 0 && chunk < chunks && p < b.passes) {
+            const bool odd = ((b.color + p) & 1) != 0;
+            const int ylo = ya == 0 ? 1 : ya + 1 + p, yhi = yb == ny ? ny - 1 : yb - 1 - p;
+            const int zlo = za == 0 ? 1 : za + 1 + p, zhi = zb == nz ? nz - 1 : zb - 1 - p;
+            const int x = 1 + chunk * kSorChunk, left = nx - 1 - x;
+            const int y = odd ? y1c : y0c, z = odd ? z1c : z0c;
+            if (r0 < rows && y >= ylo && y < yhi && z >= zlo && z < zhi)
+                sweep(u + (odd ? u1 : u0) + x, fl + (odd ? f1 : f0) + x, left);
+            for (int r = r0 + b.slot_threads; r < rows; r += b.slot_threads) {
+                int ry, rz;
+                row_of(r, odd, ry, rz);
+                if (ry >= ylo && ry < yhi && rz >= zlo && rz < zhi)
+                    sweep(u + u_at(ry, rz) + x, fl + f_at(ry, rz) + x, left);
+            }
+        }
+        if (++chunk == period) {
+            chunk = 0;
+            p += b.slots;
+        }
+        __syncthreads();
+    }
+    // owned rows, with the grid's faces where the block touches them
+    const int oy = y0 == 1 ? 0 : y0, py = y1 == ny - 1 ? ny : y1;
+    const int oz = z0 == 1 ? 0 : z0, pz = z1 == nz - 1 ? nz : z1;
+    runs(oy, py, oz, pz, ya, za, ey, [&](int at, uint32_t) { return u[at]; },
+         [&](int, uint32_t o, float v) { out[o * b.out_mul] = v; });
+}
+
+// Packed Vec3 fields to one array per component.
+__global__ void k_sor_planes(const float *__restrict__ a, const float *__restrict__ f, size_t n,
+                             float *__restrict__ pa, float *__restrict__ pf) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+#pragma unroll
+    for (size_t k = 0; k < 3; ++k) {
+        pa[k * n + i] = a[3 * i + k];
+        pf[k * n + i] = f[3 * i + k];
     }
 }
 
@@ -419,11 +612,160 @@ vg_status zero_fill(void *p, size_t bytes, hipStream_t s) {
                   (uint8_t *)p, bytes);
 }
 
-// Exposed to the multigrid driver.
+// How `passes` colour passes over a grid are dealt to k_sor_block launches;
+// by == 0: they are not (rows too long for the LDS).
+struct SorPlan {
+    int by = 0, bz = 0, passes = 0, slots = 0, slot_threads = 0, threads = 0;
+    size_t lds = 0;
+    double us = 0.0;  // estimated time of all passes
+};
+
+// Chooses among a grid's plans by an estimate of their time from what was
+// measured: 3 us to start a launch, staging and writing back at 14 bytes a
+// nanosecond, and per tick kSorChunk steps of 160 cycles, or 85 per wave
+// that shares its SIMD, and 400 for the barrier and the chunk's first reads.
+// Workgroups beyond what the 256 CUs hold at once follow in rounds.
+static SorPlan sor_plan(const vg_grid_desc &g, uint32_t total, bool scratch) {
+    const int nx = (int)g.np[0], ny = (int)g.np[1], nz = (int)g.np[2], iy = ny - 2, iz = nz - 2;
+    const int chunks = (nx - 2 + kSorChunk - 1) / kSorChunk;
+    SorPlan best;
+    auto consider = [&](int by, int bz, int passes, bool whole) {
+        const int halo = whole ? 1 : passes;
+        const int ey = std::min(ny, by + 2 * halo), ez = std::min(nz, bz + 2 * halo);
+        // kSorChunk floats behind the last row: see the kernel's reads
+        const size_t lds = (((size_t)ey * ez + (size_t)(ey - 2) * (ez - 2)) * nx +
+                            2 * kSorChunk) * sizeof(float);
+        if (lds > kSorLdsBytes) return;
+        SorPlan q;
+        q.by = by;
+        q.bz = bz;
+        q.passes = passes;
+        q.lds = lds;
+        const int rows = (ey - 1) / 2 * (ez - 2);
+        q.slot_threads = std::min(kSorThreads, (rows + 63) / 64 * 64);
+        q.slots = std::max(1, std::min(std::min(chunks, passes), kSorThreads / q.slot_threads));
+        // the staging wants every load it can have in flight, the ticks no
+        // more waves at their barriers than sweep rows
+        const int busy = q.slots * q.slot_threads;
+        q.threads = whole ? std::max(256, busy) : kSorThreads;
+        const int groups = 3 * ((iy + by - 1) / by) * ((iz + bz - 1) / bz);
+        const int fit = std::min(2, (int)(kSorLdsBytes / lds)), share = groups > 256 ? fit : 1;
+        const int rounds = (groups + 256 * fit - 1) / (256 * fit);
+        const int period = std::max(chunks, q.slots);
+        const int ticks = (passes - 1) / q.slots * period + (passes - 1) % q.slots + chunks;
+        const double step = std::max(160.0, 85.0 * share * ((busy / 64 + 3) / 4)) *
+                            ((rows + q.slot_threads - 1) / q.slot_threads);
+        const double group_us = lds * 7e-5 * share + ticks * (400.0 + kSorChunk * step) / 2400.0;
+        q.us = (3.0 + rounds * group_us) * std::ceil((double)total / passes) + (whole ? 0.0 : 6.0);
+        if (best.by == 0 || q.us < best.us) best = q;
+    };
+    consider(iy, iz, (int)total, true);
+    // one wave per SIMD or fewer: nothing is faster than a single launch
+    if (best.by && (size_t)iy * iz <= 512) return best;
+    const int sizes[] = {4, 5, 6, 7, 8, 9, 10, 11, 12, 14, 16, 20, 24, 32};
+    if (scratch)
+        for (int passes : {2, 4, 6, 8})
+            for (int by : sizes)
+                for (int bz : sizes)
+                    if (passes <= (int)total && by <= iy && bz <= iz)
+                        consider(by, bz, passes, false);
+    return best;
+}
+
+// The choice takes some tens of microseconds on the host: each thread keeps
+// its last ones (a cascade has about six grids).
+static SorPlan sor_plan_kept(const vg_grid_desc &g, uint32_t total, bool scratch) {
+    struct Kept {
+        uint32_t np[3] = {0, 0, 0}, total = 0;
+        bool scratch = false;
+        SorPlan plan;
+    };
+    static thread_local Kept kept[16];
+    static thread_local unsigned next = 0;
+    for (const Kept &k : kept)
+        if (k.np[0] == g.np[0] && k.np[1] == g.np[1] && k.np[2] == g.np[2] && k.total == total &&
+            k.scratch == scratch)
+            return k.plan;
+    Kept &k = kept[next++ % 16];
+    for (int a = 0; a < 3; ++a) k.np[a] = g.np[a];
+    k.total = total;
+    k.scratch = scratch;
+    k.plan = sor_plan(g, total, scratch);
+    return k.plan;
+}
+
+// Exposed to the multigrid driver.  scratch: 9 floats per point, or null for
+// an allocation on the stream.
 vg_status sor_solve(const vg_grid_desc &g, float *soln, const float *lap, uint32_t steps,
-                    hipStream_t s) {
+                    hipStream_t s, float *scratch) {
     if (g.np[0] < 3 || g.np[1] < 3 || g.np[2] < 3) return VG_OK;  // no interior
+    if (steps == 0) return VG_OK;
     const SorCoef c = sor_coef(g);
+    const size_t n = capacity(g);
+    // a stream under capture takes no allocation: without scratch, its grids
+    // that do not fit one workgroup keep the row kernels
+    bool may = scratch != nullptr;
+    if (!scratch) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+        if (hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
+        else may = capture == hipStreamCaptureStatusNone;
+    }
+    // (an odd row stride and 32-bit offsets: see k_sor_block)
+    const bool fits = (g.np[0] & 1u) && steps < (1u << 24) && 3 * n < (size_t(1) << 31);
+    const SorPlan plan = fits ? sor_plan_kept(g, 2 * steps, may) : SorPlan();
+    const bool whole = plan.by > 0 && plan.passes == (int)(2 * steps) &&
+                       plan.by == (int)g.np[1] - 2 && plan.bz == (int)g.np[2] - 2;
+    float *own = nullptr;
+    if (plan.by > 0 && !whole && !scratch) {
+        // (no memory for it: the row kernels need none)
+        if (salloc((void **)&own, 9 * n * sizeof(float), s) == VG_OK) scratch = own;
+        else (void)hipGetLastError();
+    }
+    if (plan.by > 0 && (whole || scratch)) {
+        VG_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_sor_block),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSorLdsBytes));
+        SorBlock b;
+        b.nx = (int)g.np[0];
+        b.ny = (int)g.np[1];
+        b.nz = (int)g.np[2];
+        b.by = plan.by;
+        b.bz = plan.bz;
+        b.slots = plan.slots;
+        b.slot_threads = plan.slot_threads;
+        const dim3 grid(ceil_div(g.np[1] - 2, plan.by), ceil_div(g.np[2] - 2, plan.bz), 3);
+        const dim3 block(plan.threads);
+        vg_status st = VG_OK;
+        if (whole) {
+            b.in_mul = b.out_mul = b.f_mul = 3;
+            b.in_comp = b.out_comp = b.f_comp = 1;
+            // about a millisecond a launch at most
+            constexpr uint32_t kMost = 1024;
+            for (uint32_t done = 0; done < 2 * steps && st == VG_OK; done += kMost) {
+                b.passes = (int)std::min(kMost, 2 * steps - done);
+                b.color = 0;
+                st = launch("vg_sor_block", k_sor_block, grid, block, plan.lds, s, b,
+                            (const float *)soln, soln, lap, c);
+            }
+            return st;
+        }
+        float *from = scratch, *to = scratch + 3 * n, *f = scratch + 6 * n;
+        st = launch("vg_sor_planes", k_sor_planes, dim3(ceil_div(n, 256)), dim3(256), 0, s,
+                    (const float *)soln, lap, n, from, f);
+        b.in_mul = b.f_mul = 1;
+        b.in_comp = b.f_comp = n;
+        for (uint32_t done = 0; done < 2 * steps && st == VG_OK; done += (uint32_t)b.passes) {
+            b.passes = (int)std::min<uint32_t>((uint32_t)plan.passes, 2 * steps - done);
+            b.color = (int)(done & 1u);
+            const bool last = done + (uint32_t)b.passes == 2 * steps;
+            b.out_mul = last ? 3 : 1;
+            b.out_comp = last ? 1 : n;
+            st = launch("vg_sor_block", k_sor_block, grid, block, plan.lds, s, b,
+                        (const float *)from, last ? soln : to, (const float *)f, c);
+            std::swap(from, to);
+        }
+        if (own) sfree(own, s);
+        return st;
+    }
     const uint32_t rows_half = (g.np[1] - 1) / 2 + 1;
     const bool split = (size_t)rows_half * (g.np[2] - 2) >= kSorSplitRows;
     const dim3 grid(ceil_div(rows_half, split ? kSorRowsPerWave : 64u), g.np[2] - 2);
@@ -539,7 +881,7 @@ VG_API vg_status vg_sor_solve(const vg_grid_desc *g, float *soln, const float *l
         if (g->np[2] > m) m = g->np[2];
         n = 2 * m;
     }
-    return sor_solve(*g, soln, lap, n, (hipStream_t)s);
+    return sor_solve(*g, soln, lap, n, (hipStream_t)s, nullptr);
 }
 
 VG_API vg_status vg_curl(const vg_grid_desc *g, const float *a, float *out, vg_stream s) {
