@@ -1,0 +1,34 @@
+"""The direct sums' fine blocks (128 queries by whole tiles of 256 sources):
+the edges of the query block, of a tile and of a wave's quarter of it, one
+source and one query, and the split over several tiles, against the CPU
+oracle; strided vortons with their own sizes included."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+F32 = np.float32
+
+
+@pytest.mark.parametrize("policy", [0, 1])
+@pytest.mark.parametrize("n,nq", [(1, 1), (63, 127), (64, 128), (65, 129), (255, 64), (256, 1),
+                                  (257, 300), (1023, 513), (4097, 4095), (12345, 77)])
+def test_fine_blocks(vg, oracle, n, nq, policy):
+    print(f"[case] direct sum, {n} vortons, {nq} queries, policy {policy}", flush=True)
+    rng = np.random.default_rng(n + nq)
+    rec = rng.normal(size=(n, 18)).astype(F32)
+    rec[:, 13] = rng.uniform(0.05, 0.3, n)
+    q = rng.normal(size=(nq, 4)).astype(F32)
+    d, dq = vg.DeviceArray.from_numpy(rec), vg.DeviceArray.from_numpy(q)
+    v = vg.Vortons()
+    v.pos, v.angvel, v.size = d.ptr.value, d.offset(9).value, d.offset(13).value
+    v.stride, v.n, v.uniform_size = 18, n, 0.0
+    pos, om, size = (np.ascontiguousarray(a) for a in (rec[:, 0:3], rec[:, 9:12], rec[:, 13]))
+    pts = np.ascontiguousarray(q[:, :3])
+    for gpu, cpu in ((vg.direct_velocity, oracle.direct_velocity),
+                     (vg.direct_vecpot, oracle.direct_vecpot)):
+        out = vg.DeviceArray.zeros((nq, 3))
+        gpu(v, dq, nq, out, 1.3, 0.7, policy, q_stride=4)
+        vg.synchronize()
+        want = cpu(pos, om, size, pts, 1.3, 0.7, policy=policy, threads=8)
+        # FP32 terms of random sign summed in another order
+        assert np.linalg.norm(out.numpy() - want) <= 1e-5 * np.linalg.norm(want)

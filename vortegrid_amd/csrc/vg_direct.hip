@@ -9,6 +9,7 @@
 // plain FP32 partial per tile and folds it into a Kahan-compensated total
 // once per tile.  Small problems split the source range over blockIdx.y and
 // reduce the partials in fixed order (deterministic).
+#include <algorithm>
 #include <mutex>
 #include <string>
 
@@ -130,6 +131,78 @@ __global__ __launch_bounds__(kBlock) void k_direct(const float4 *__restrict__ A,
             o[0] = sum[k].x * circ; o[1] = sum[k].y * circ; o[2] = sum[k].z * circ;
         }
     }
+}
+
+// The same sum for sizes whose (512 queries, 1024 sources) blocks above leave
+// most of the chip idle.  A workgroup owns 64 kSmallQPT queries, its four
+// waves take a quarter of each 256-source tile and add their shares through
+// LDS at the end, so a block is 128 queries by one tile: 4096 queries of 4096
+// vortons make 512 workgroups instead of 32 (111 -> 22 us with the launches
+// around it).  Sources are prepared as they are staged, which spares the
+// packing launch.  Writes partials only: the reduction's launch orders them
+// after every read of the vortons, as the packed copy does above.
+constexpr int kSmallQPT = 2, kSmallQueries = 64 * kSmallQPT;
+
+template <int POLICY, int VECPOT, int GRID>
+__global__ __launch_bounds__(kBlock) void k_direct_small(SourceView sv, size_t n, float spread,
+                                                         size_t chunk, QueryView qv,
+                                                         float *__restrict__ partial) {
+    __shared__ float4 sA[kTile], sB[kTile];
+    __shared__ float share[4][3 * kSmallQueries];
+    const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+    const size_t q0 = (size_t)blockIdx.x * kSmallQueries + lane;
+    float3 q[kSmallQPT], sum[kSmallQPT], comp[kSmallQPT];
+#pragma unroll
+    for (int k = 0; k < kSmallQPT; ++k) {
+        const size_t qi = q0 + (size_t)k * 64;
+        q[k] = qi < qv.nq ? query_at<GRID>(qv, qi) : make_float3(0.f, 0.f, 0.f);
+        sum[k] = comp[k] = make_float3(0.f, 0.f, 0.f);
+    }
+    const size_t s0 = (size_t)blockIdx.y * chunk;
+    const size_t s1 = s0 + chunk < n ? s0 + chunk : n;
+    for (size_t t0 = s0; t0 < s1; t0 += kTile) {
+        const int cnt = (int)(s1 - t0 < (size_t)kTile ? s1 - t0 : (size_t)kTile);
+        __syncthreads();
+        if ((int)threadIdx.x < cnt) {
+            const size_t i = t0 + threadIdx.x;
+            const float *p = sv.pos + i * sv.stride, *w = sv.angvel + i * sv.stride;
+            const float sz = sv.size ? sv.size[i * sv.stride] : sv.usize;
+            float4 a, b;
+            prepare_source(make_float4(p[0], p[1], p[2], sz), make_float4(w[0], w[1], w[2], 0.f),
+                           spread, a, b);
+            sA[threadIdx.x] = a;
+            sB[threadIdx.x] = b;
+        }
+        __syncthreads();
+        float3 part[kSmallQPT];
+#pragma unroll
+        for (int k = 0; k < kSmallQPT; ++k) part[k] = make_float3(0.f, 0.f, 0.f);
+        const int j0 = wave * (kTile / 4), j1 = min(cnt, j0 + kTile / 4);
+#pragma unroll 4
+        for (int j = j0; j < j1; ++j) {
+            const float4 a = sA[j], b = sB[j];
+#pragma unroll
+            for (int k = 0; k < kSmallQPT; ++k) {
+                if (VECPOT) pair_vecpot<POLICY>(part[k], q[k], a, b);
+                else pair_velocity<POLICY>(part[k], q[k], a, b);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kSmallQPT; ++k) kahan_add(sum[k], comp[k], part[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < kSmallQPT; ++k) {
+        float *o = share[wave] + 3 * (lane + 64 * k);
+        o[0] = sum[k].x;
+        o[1] = sum[k].y;
+        o[2] = sum[k].z;
+    }
+    __syncthreads();
+    const size_t first = 3 * (size_t)blockIdx.x * kSmallQueries;
+    for (int i = (int)threadIdx.x; i < 3 * kSmallQueries; i += kBlock)
+        if (first + i < 3 * qv.nq)
+            partial[(size_t)blockIdx.y * 3 * qv.nq + first + i] =
+                (share[0][i] + share[1][i]) + (share[2][i] + share[3][i]);
 }
 
 // Fixed-order Kahan reduction of the source-split partials.
@@ -254,7 +327,27 @@ vg_status run_direct(const vg_vortons *v, QueryView qv, float spread, float circ
     chunk = (chunk + kTile - 1) / kTile * kTile;
     nsplit = (uint32_t)((n + chunk - 1) / chunk);
     const size_t src_bytes = n * sizeof(float4);
-    const size_t part_bytes = nsplit > 1 ? (size_t)nsplit * qv.nq * 3 * sizeof(float) : 0;
+    size_t part_bytes = nsplit > 1 ? (size_t)nsplit * qv.nq * 3 * sizeof(float) : 0;
+    // Fewer than 1024 workgroups leave SIMDs idle or unevenly loaded: finer
+    // blocks then (4096 x 4096: 32 workgroups, 111 -> 22 us; 50781 x 8464:
+    // 833).  Not where either's buffers would outgrow the fixed scratch: what
+    // it refuses stays refused, and the rule is the same with and without it,
+    // so that both forms give the same bits.
+    bool small = false;
+    const size_t split_queries = ceil_div(qv.nq, (size_t)kSmallQueries);
+    if ((size_t)qblocks * nsplit < 1024) {
+        const size_t tiles = ceil_div(n, (size_t)kTile);
+        const size_t want = (2048 + split_queries - 1) / split_queries;
+        const size_t per = (tiles + std::min(tiles, want) - 1) / std::min(tiles, want);
+        const size_t ns = (tiles + per - 1) / per, bytes = ns * qv.nq * 3 * sizeof(float);
+        if (ns < 65536 && 2 * align256(src_bytes) + align256(std::max(bytes, part_bytes)) <=
+                              kFixedScratchBytes) {
+            small = true;
+            chunk = per * kTile;
+            nsplit = (uint32_t)ns;
+            part_bytes = bytes;
+        }
+    }
     float4 *A = nullptr, *B = nullptr;
     float *partial = nullptr;
     if (fixed.base) {
@@ -271,9 +364,23 @@ vg_status run_direct(const vg_vortons *v, QueryView qv, float spread, float circ
         if (part_bytes)
             partial = reinterpret_cast<float *>(fixed.base + 2 * align256(src_bytes));
     } else {
-        VG_TRY(salloc((void **)&A, src_bytes, s));
-        VG_TRY(salloc((void **)&B, src_bytes, s));
+        if (!small) {
+            VG_TRY(salloc((void **)&A, src_bytes, s));
+            VG_TRY(salloc((void **)&B, src_bytes, s));
+        }
         if (part_bytes) VG_TRY(salloc((void **)&partial, part_bytes, s));
+    }
+    if (small) {
+        auto kern = policy == VG_RSQRT_REFERENCE
+                        ? k_direct_small<VG_RSQRT_REFERENCE, VECPOT, GRID>
+                        : k_direct_small<VG_RSQRT_ACCURATE, VECPOT, GRID>;
+        vg_status st = launch(name, kern, dim3((uint32_t)split_queries, nsplit), dim3(kBlock), 0, s,
+                              source_view(v), n, spread, chunk, qv, partial);
+        if (st == VG_OK)
+            st = launch("vg_direct_reduce", k_reduce_split, dim3(ceil_div(qv.nq, 256)), dim3(256),
+                        0, s, (const float *)partial, nsplit, qv.nq, circ, out);
+        if (!fixed.base) sfree(partial, s);
+        return st;
     }
     VG_TRY(launch("vg_pack_sources", k_pack_sources, dim3(ceil_div(n, 256)), dim3(256), 0, s,
                   source_view(v), n, spread, A, B));
