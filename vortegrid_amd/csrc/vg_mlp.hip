@@ -519,8 +519,22 @@ __device__ __forceinline__ bf16x8 pack8(const float *v) {
     return r;
 }
 
+// (a, b) -> (a's lanes 0-31 and b's lanes 0-31, a's lanes 32-63 and b's lanes
+// 32-63): the upper half of a changes places with the lower half of b.
+__device__ __forceinline__ void swap_halves(uint32_t &a, uint32_t &b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+
 // One wave = one brick; for every accepted cluster of the masked layers the
-// brick's 64 points form one batch of 64 pairs (two 32-column tiles).
+// brick's 64 points form one batch of 64 pairs (two 32-column tiles).  Each
+// lane forms the 16 features of its own point's pair; the lane groups of the
+// first layer's operands (features 0-7 and 8-15 of columns 0-31, then of
+// columns 32-63) come from exchanging half-waves.  (With every lane forming
+// the features of its two columns, and picking its eight by lane group, a
+// pair took 2650 instructions instead of 1700, 360 of them selects and 300
+// moves of the selects' masks: 1M vortons, near_k 1, 62 -> 43 ms.)
 __global__ __launch_bounds__(256, 2) void k_mlp_grid(const vg::TreeView tv, vg_grid_desc g,
                                                   MlpGridParams mp,
                                                   const __bf16 *__restrict__ packed,
@@ -558,13 +572,11 @@ __global__ __launch_bounds__(256, 2) void k_mlp_grid(const vg::TreeView tv, vg_g
     if (brick >= mp.nbricks) return;
     ClusterStage &S = stage[wave];
     const uint32_t lane = threadIdx.x & 63;
-    const uint32_t col = lane & 31, grp = lane >> 5;
+    const uint32_t grp = lane >> 5;
     const uint32_t bb[3] = {brick % mp.nb[0], (brick / mp.nb[0]) % mp.nb[1],
                             brick / (mp.nb[0] * mp.nb[1])};
     bool valid;
     const float3 qo = brick_point(g, bb, lane, &valid);  // this lane's own point
-    const float3 qa = brick_point(g, bb, col, nullptr);       // pair column tile 0
-    const float3 qb = brick_point(g, bb, col + 32, nullptr);  // pair column tile 1
     int cl0[3], cl1[3];
     brick_cells(g, bb, cl0, cl1);
     const bf16x8 *W8 = (const bf16x8 *)wts;
@@ -618,10 +630,17 @@ __global__ __launch_bounds__(256, 2) void k_mlp_grid(const vg::TreeView tv, vg_g
                     const float4 cp = S.P[j], cw = S.W[j];
                     const float4 a0 = S.M0[j], a1 = S.M1[j], a2 = S.M2[j];
                     // layer-1 inputs: lane group 0 holds features 0..7, group 1 8..15
-                    float fa[kIn], fb[kIn];
-                    cluster_features(fa, nullptr, qa, cp, cw, a0, a1, a2, inv_h);
-                    cluster_features(fb, nullptr, qb, cp, cw, a0, a1, a2, inv_h);
-                    const bf16x8 xa = pack8(fa + 8 * grp), xb = pack8(fb + 8 * grp);
+                    float fo[kIn], Bo[9];
+                    cluster_features(fo, Bo, qo, cp, cw, a0, a1, a2, inv_h);
+                    union {
+                        bf16x8 v;
+                        uint32_t u[4];
+                    } lo8, hi8;
+                    lo8.v = pack8(fo);
+                    hi8.v = pack8(fo + 8);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) swap_halves(lo8.u[t], hi8.u[t]);
+                    const bf16x8 xa = lo8.v, xb = hi8.v;
                     auto bias16 = [&](int layer, int r) {
                         f32x16 b;
 #pragma unroll
@@ -684,12 +703,11 @@ __global__ __launch_bounds__(256, 2) void k_mlp_grid(const vg::TreeView tv, vg_g
                     float o[3];
 #pragma unroll
                     for (int v = 0; v < 3; ++v) {
-                        const float other = __shfl(y1[v], (int)col, 64);
-                        o[v] = (lane < 32 ? y0[v] : other) + bias[3 * kHid + v];
+                        uint32_t a = __float_as_uint(y0[v]), b = __float_as_uint(y1[v]);
+                        swap_halves(a, b);
+                        o[v] = __uint_as_float(a) + bias[3 * kHid + v];
                     }
                     // correction = scale * B c at this lane's own point
-                    float fo[kIn], Bo[9];
-                    cluster_features(fo, Bo, qo, cp, cw, a0, a1, a2, inv_h);
                     const float sc = correction_scale(cp, cw, inv_h);
                     corr.x += (Bo[0] * o[0] + Bo[1] * o[1] + Bo[2] * o[2]) * sc;
                     corr.y += (Bo[3] * o[0] + Bo[4] * o[1] + Bo[5] * o[2]) * sc;
