@@ -533,8 +533,8 @@ __device__ __forceinline__ void swap_halves(uint32_t &a, uint32_t &b) {
 // first layer's operands (features 0-7 and 8-15 of columns 0-31, then of
 // columns 32-63) come from exchanging half-waves.  (With every lane forming
 // the features of its two columns, and picking its eight by lane group, a
-// pair took 2650 instructions instead of 1700, 360 of them selects and 300
-// moves of the selects' masks: 1M vortons, near_k 1, 62 -> 43 ms.)
+// pair took 2650 instructions instead of 1770, 360 of them selects and 300
+// moves of the selects' masks: 65,536 vortons, near_k 1, 9.31 -> 7.00 ms.)
 __global__ __launch_bounds__(256, 2) void k_mlp_grid(const vg::TreeView tv, vg_grid_desc g,
                                                   MlpGridParams mp,
                                                   const __bf16 *__restrict__ packed,
