@@ -18,15 +18,16 @@
 //
 // Everything that multiplies matrices runs on BF16 MFMA with FP32
 // accumulation:
-//   * training: k_gemm (v_mfma_f32_16x16x32_bf16, 64x64 block tiles) for the
-//     forward and backward products, elementwise GELU / loss / bias-gradient
-//     kernels, Adam;
+//   * training: k_mlp_pass (v_mfma_f32_16x16x32_bf16), forward and backward of
+//     64 rows in one workgroup, and k_mlp_sum, the sums over the workgroups
+//     with Adam's update;
 //   * inference at grid points: k_mlp_grid, one wave per 4x4x4 brick, one
 //     accepted cluster at a time: the 64 (point, cluster) pairs of the brick
 //     form the batch, all four layers run on v_mfma_f32_32x32x16_bf16 with
 //     the weights in LDS, and the hidden activations stay in registers
 //     between layers (the output layout of one product is consumed directly
 //     as the input layout of the next; the weights are packed in that order).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -42,6 +43,7 @@ vg_status mac_velocity_grid(const vg_tree *t, const vg_grid_desc *g, int near_k,
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -91,257 +93,349 @@ __device__ __forceinline__ float gelu_grad(float z) {
     return 0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * kGeluC * (1.0f + 3.0f * kGeluA * z * z);
 }
 
-// ------------------------------------------------------------------ GEMM
-// C[M][N] (ldc) = sum_k opA(m, k) opB(k, n) with opA(m, k) = TA ? A[k][m] :
-// A[m][k] and opB(k, n) = TB ? B[n][k] : B[k][n].  FP32 in memory, operands
-// rounded to bf16 when staged to LDS, FP32 accumulation.  Block = 4 waves,
-// 64x64 tile, each wave 32x32 = 2x2 MFMA 16x16x32 tiles, K step 32.
-// blockIdx.z splits K into chunks of kc: chunk z writes its partial product
-// to C + z * M * ldc (reduced afterwards by k_reduce_split).
-template <bool TA, bool TB>
-__global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, const float *__restrict__ A,
-                                              int lda, const float *__restrict__ B, int ldb,
-                                              float *__restrict__ C, int ldc, int kc) {
-    __shared__ __attribute__((aligned(16))) __bf16 As[64][40];
-    __shared__ __attribute__((aligned(16))) __bf16 Bs[64][40];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int m0 = blockIdx.x * 64, n0 = blockIdx.y * 64;
-    const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-    const int kb = blockIdx.z * kc, ke = min(K, kb + kc);
-    C += (size_t)blockIdx.z * M * ldc;
-    f32x4 acc[2][2];
+// ------------------------------------------------------------------ training
+// One Adam update of parameter i; the gradient is gi.
+struct Adam {
+    float *p, *m1, *m2;
+    float lr, b1, b2, eps, bc1, bc2;
+};
+__device__ __forceinline__ void adam_update(const Adam &o, int i, float gi) {
+    const float a = o.b1 * o.m1[i] + (1.0f - o.b1) * gi;
+    const float v = o.b2 * o.m2[i] + (1.0f - o.b2) * gi * gi;
+    o.m1[i] = a;
+    o.m2[i] = v;
+    o.p[i] -= o.lr * (a / o.bc1) / (sqrtf(v / o.bc2) + o.eps);
+}
+
+constexpr int kRows = 64;         // rows of the batch per tile
+constexpr int kRowTiles = 256;    // workgroups of the gradient: one per CU
+constexpr int kLdw = kHid + 8;    // LDS row of a 64-wide operand: 16-byte aligned, off the banks
+constexpr int kLdn = 32 + 8;      // of a 16-wide operand, zero-padded to one 32-wide product step
+constexpr int kSlab = kPadParams + 1;  // a workgroup's gradients and its loss
+
+// Operands in LDS, rounded to bf16.  "T" is the transpose of what precedes
+// it: a product reads eight consecutive values along its contraction.
+struct FwdLds {
+    __bf16 w1t[kHid][kLdn], w2t[kHid][kLdw], w3t[kHid][kLdw], w4t[kOutPad][kLdw];
+    __bf16 r0[kRows][kLdw], r1[kRows][kLdw];  // activations of alternate layers, by row
+    float y[kRows][kOutPad + 1];
+    float b[3 * kHid + kOutPad];
+};
+struct GradLds : FwdLds {
+    __bf16 w2[kHid][kLdw], w3[kHid][kLdw], w4[kHid][kLdn];
+    __bf16 xt[kIn][kLdw], a1t[kHid][kLdw], a2t[kHid][kLdw], a3t[kHid][kLdw];
+    __bf16 dyt[kOutPad][kLdw], d0t[kHid][kLdw], d1t[kHid][kLdw];
+    float bias_sum[2][kHid];
+};
+
+// acc += A B over kdim: A [row][k] from row m0, B [column][k] from column n0,
+// I x J tiles of 16x16.
+template <int I, int J, int LA, int LB>
+__device__ __forceinline__ void tile_product(f32x4 (&acc)[I][J], const __bf16 (*A)[LA], int m0,
+                                             const __bf16 (*B)[LB], int n0, int kdim) {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    for (int k = 0; k < kdim; k += 32) {
+        bf16x8 a[I], b[J];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < I; ++i) a[i] = *(const bf16x8 *)&A[m0 + i * 16 + r][k + g * 8];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = kb; k0 < ke; k0 += 32) {
-        for (int e = tid; e < 64 * 32; e += 256) {
-            const int mm = TA ? (e & 63) : (e >> 5), kk = TA ? (e >> 6) : (e & 31);
-            const int gm = m0 + mm, gk = k0 + kk;
-            float v = 0.f;
-            if (gm < M && gk < ke) v = TA ? A[(size_t)gk * lda + gm] : A[(size_t)gm * lda + gk];
-            As[mm][kk] = (__bf16)v;
-        }
-        for (int e = tid; e < 64 * 32; e += 256) {
-            const int nn = TB ? (e >> 5) : (e & 63), kk = TB ? (e & 31) : (e >> 6);
-            const int gn = n0 + nn, gk = k0 + kk;
-            float v = 0.f;
-            if (gn < N && gk < ke) v = TB ? B[(size_t)gn * ldb + gk] : B[(size_t)gk * ldb + gn];
-            Bs[nn][kk] = (__bf16)v;
-        }
-        __syncthreads();
-        const int r = lane & 15, g = lane >> 4;
-        bf16x8 a[2], b[2];
+        for (int j = 0; j < J; ++j) b[j] = *(const bf16x8 *)&B[n0 + j * 16 + r][k + g * 8];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) a[i] = *(const bf16x8 *)&As[wm + i * 16 + r][g * 8];
+        for (int i = 0; i < I; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) b[j] = *(const bf16x8 *)&Bs[wn + j * 16 + r][g * 8];
+            for (int j = 0; j < J; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+}
+template <int I, int J>
+__device__ __forceinline__ void tile_zero(f32x4 (&acc)[I][J]) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+        for (int j = 0; j < J; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+// Column sums of a wave's 32x32 tile, per lane and column tile.
+__device__ __forceinline__ void tile_colsum(float (&sum)[2], const f32x4 (&d)[2][2]) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-        __syncthreads();
+            for (int v = 0; v < 4; ++v) sum[j] += d[i][j][v];
+}
+
+// Forward pass, and with GRAD the loss and the gradients, of the tiles
+// blockIdx.x, blockIdx.x + gridDim.x, ... of kRows rows; four waves, each a
+// 32x32 quarter of every 64x64 product.
+//
+// Loss of the correction vectors B c (B = identity when null) against T:
+// dY = 2 B^T (B c - T) / (3 rows).  Z = A_prev W + b and A = gelu(Z) go down,
+// dZ = dA gelu'(Z), dW = A_prev^T dZ, db = column sums of dZ and
+// dA_prev = dZ W^T up; products with bf16 operands and FP32 accumulators, all
+// else in FP32.  The pre-activations and the weights' gradients stay in
+// registers, what a product reads is in LDS, and the rows are read once:
+// 20 KB of LDS traffic per product is the work, the barriers between the
+// eleven products are the time.  Each workgroup writes its gradients and its
+// loss to a slab of its own, summed in a fixed order by k_mlp_sum.  (One
+// launch per product, activation and column sum was bound by 26 launches and
+// serial sums over the slabs: the gradients of 4,096 rows, 334 -> 63 us with
+// their copy to the host, 20 of them on the device; an Adam step on 2,048
+// rows, 215 -> 20 us; of 1M rows forward, 1290 -> 121 us.)
+template <bool GRAD>
+__global__ __launch_bounds__(256) void k_mlp_pass(const float *__restrict__ P,
+                                                  const float *__restrict__ X,
+                                                  const float *__restrict__ Bm,
+                                                  const float *__restrict__ T, uint32_t rows,
+                                                  float scale, float *__restrict__ out) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    GradLds &L = *(GradLds *)lds;  // only the FwdLds part is there without GRAD
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+    const int r16 = lane & 15, g4 = (lane >> 4) * 4;
+
+    for (int e = tid; e < kHid * 32; e += 256) {
+        const int k = e >> 6, n = e & 63;  // W1 [k][n], zero for the padding of k
+        L.w1t[n][k] = (__bf16)(k < kIn ? P[kOffW1 + (k < kIn ? e : 0)] : 0.f);
     }
+#pragma unroll 4
+    for (int e = tid; e < kHid * kHid; e += 256) {
+        const int k = e >> 6, n = e & 63;
+        const __bf16 v2 = (__bf16)P[kOffW2 + e], v3 = (__bf16)P[kOffW3 + e];
+        L.w2t[n][k] = v2;
+        L.w3t[n][k] = v3;
+        if (GRAD) {
+            L.w2[k][n] = v2;
+            L.w3[k][n] = v3;
+        }
+    }
+    for (int e = tid; e < kHid * kOutPad; e += 256) {
+        const int k = e >> 4, n = e & 15;
+        const __bf16 v = (__bf16)P[kOffW4 + e];
+        L.w4t[n][k] = v;
+        if (GRAD) {
+            L.w4[k][n] = v;
+            L.w4[k][16 + n] = (__bf16)0.f;
+        }
+    }
+    if (tid < kHid) {
+        L.b[tid] = P[kOffB1 + tid];
+        L.b[kHid + tid] = P[kOffB2 + tid];
+        L.b[2 * kHid + tid] = P[kOffB3 + tid];
+        if (tid < kOutPad) L.b[3 * kHid + tid] = P[kOffB4 + tid];
+    }
+    if (GRAD)
+        for (int e = tid; e < kOutPad * kLdw; e += 256) (&L.dyt[0][0])[e] = (__bf16)0.f;
+
+    f32x4 gw1[1][1], gw2[2][2], gw3[2][2], gw4[1][1];
+    float gb1[2] = {0.f, 0.f}, gb2[2] = {0.f, 0.f}, gb3[2] = {0.f, 0.f};
+    float gb4[kOut] = {0.f, 0.f, 0.f}, loss = 0.f;
+    tile_zero(gw1);
+    tile_zero(gw2);
+    tile_zero(gw3);
+    tile_zero(gw4);
+
+    for (size_t r0 = (size_t)blockIdx.x * kRows; r0 < rows; r0 += (size_t)gridDim.x * kRows) {
+        const uint32_t live = (uint32_t)(rows - r0 < kRows ? rows - r0 : kRows);
+        f32x4 z1[2][2], z2[2][2], z3[2][2];
+        __syncthreads();  // the last tile's products have read r0 and xt
+#pragma unroll
+        for (int q = 0; q < kRows * 32 / 256; ++q) {
+            const int e = tid + q * 256, row = e >> 5, k = e & 31;
+            const bool in = k < kIn && (uint32_t)row < live;
+            const __bf16 v = (__bf16)(in ? X[(r0 + (in ? row : 0)) * kIn + (in ? k : 0)] : 0.f);
+            L.r0[row][k] = v;
+            if (GRAD && k < kIn) L.xt[k][row] = v;
+        }
+        __syncthreads();
+        // Z = acc + b, A = gelu(Z) into dst by row and, for the gradient, into
+        // dt by column (rows beyond the batch as zeros: they add nothing)
+        auto activate = [&](f32x4(&z)[2][2], int layer, __bf16(*dst)[kLdw], __bf16(*dt)[kLdw]) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int n = wn + j * 16 + r16;
+                const float bias = L.b[layer * kHid + n];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int m = wm + i * 16 + g4;
+                    bf16x4 t;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        z[i][j][v] += bias;
+                        const __bf16 act = (__bf16)gelu(z[i][j][v]);
+                        dst[m + v][n] = act;
+                        t[v] = (uint32_t)(m + v) < live ? act : (__bf16)0.f;
+                    }
+                    if (GRAD) *(bf16x4 *)&dt[n][m] = t;
+                }
+            }
+        };
+        tile_zero(z1);
+        tile_product(z1, L.r0, wm, L.w1t, wn, 32);
+        activate(z1, 0, L.r1, L.a1t);
+        __syncthreads();
+        tile_zero(z2);
+        tile_product(z2, L.r1, wm, L.w2t, wn, kHid);
+        activate(z2, 1, L.r0, L.a2t);
+        __syncthreads();
+        tile_zero(z3);
+        tile_product(z3, L.r0, wm, L.w3t, wn, kHid);
+        activate(z3, 2, L.r1, L.a3t);
+        __syncthreads();
+        {
+            f32x4 y[1][1];
+            tile_zero(y);
+            tile_product(y, L.r1, wave * 16, L.w4t, 0, kHid);
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                L.y[wave * 16 + g4 + v][r16] = y[0][0][v] + L.b[3 * kHid + r16];
+        }
+        __syncthreads();
+        if (!GRAD) {
+            if ((uint32_t)tid < live * kOut)
+                out[r0 * kOut + tid] = L.y[tid / kOut][tid % kOut];
+            continue;
+        }
+        if (tid < kRows) {
+            const size_t r = r0 + ((uint32_t)tid < live ? tid : 0);
+            const float y[3] = {L.y[tid][0], L.y[tid][1], L.y[tid][2]};
+            float e[3], g[3];
+            const float *b = Bm + r * 9;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                float v = y[i];
+                if (Bm) v = b[3 * i] * y[0] + b[3 * i + 1] * y[1] + b[3 * i + 2] * y[2];
+                e[i] = v - T[r * kOut + i];
+            }
+            bf16x8 d, zero;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) d[k] = zero[k] = (__bf16)0.f;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                g[k] = e[k];
+                if (Bm) g[k] = b[k] * e[0] + b[3 + k] * e[1] + b[6 + k] * e[2];
+                g[k] = (uint32_t)tid < live ? scale * g[k] : 0.f;
+                gb4[k] += g[k];
+                d[k] = (__bf16)g[k];
+                L.dyt[k][tid] = d[k];
+            }
+            if ((uint32_t)tid < live) loss += e[0] * e[0] + e[1] * e[1] + e[2] * e[2];
+            *(bf16x8 *)&L.r0[tid][0] = d;
+            *(bf16x8 *)&L.r0[tid][8] = zero;
+            *(bf16x8 *)&L.r0[tid][16] = zero;
+            *(bf16x8 *)&L.r0[tid][24] = zero;
+        }
+        __syncthreads();
+        // dZ = dA gelu'(Z) into dst by row (unless null) and dt by column
+        auto back = [&](f32x4(&d)[2][2], const f32x4(&z)[2][2], float(&gb)[2], __bf16(*dst)[kLdw],
+                        __bf16(*dt)[kLdw]) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int n = wn + j * 16 + r16;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int m = wm + i * 16 + g4;
+                    bf16x4 t;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const float dz = d[i][j][v] * gelu_grad(z[i][j][v]);
+                        d[i][j][v] = (uint32_t)(m + v) < live ? dz : 0.f;
+                        t[v] = (__bf16)d[i][j][v];
+                        if (dst) dst[m + v][n] = t[v];
+                    }
+                    *(bf16x4 *)&dt[n][m] = t;
+                }
+            }
+            tile_colsum(gb, d);
+        };
+        f32x4 d[2][2];
+        tile_zero(d);
+        tile_product(d, L.r0, wm, L.w4, wn, 32);
+        tile_product(gw4, L.a3t, wave * 16, L.dyt, 0, kRows);
+        back(d, z3, gb3, L.r1, L.d0t);
+        __syncthreads();
+        tile_zero(d);
+        tile_product(d, L.r1, wm, L.w3, wn, kHid);
+        tile_product(gw3, L.a2t, wm, L.d0t, wn, kRows);
+        back(d, z2, gb2, L.r0, L.d1t);
+        __syncthreads();
+        tile_zero(d);
+        tile_product(d, L.r0, wm, L.w2, wn, kHid);
+        tile_product(gw2, L.a1t, wm, L.d1t, wn, kRows);
+        back(d, z1, gb1, (__bf16(*)[kLdw])nullptr, L.d0t);
+        __syncthreads();
+        tile_product(gw1, L.xt, 0, L.d0t, wave * 16, kRows);
+    }
+    if (!GRAD) return;
+
+    float *o = out + (size_t)blockIdx.x * kSlab;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int gm = m0 + wm + i * 16 + (lane >> 4) * 4 + v;
-                const int gn = n0 + wn + j * 16 + (lane & 15);
-                if (gm < M && gn < N) C[(size_t)gm * ldc + gn] = acc[i][j][v];
+                const int e = (wm + i * 16 + g4 + v) * kHid + wn + j * 16 + r16;
+                o[kOffW2 + e] = gw2[i][j][v];
+                o[kOffW3 + e] = gw3[i][j][v];
             }
-}
-
-// C[m][n] = sum of the nsplit partial slabs, in slab order.
-__global__ void k_reduce_split(const float *__restrict__ part, int nsplit, int M, int N, int ldp,
-                               float *__restrict__ C, int ldc) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= M * N) return;
-    const int m = i / N, n = i % N;
-    float s = 0.f;
-    for (int z = 0; z < nsplit; ++z) s += part[(size_t)z * M * ldp + (size_t)m * ldp + n];
-    C[(size_t)m * ldc + n] = s;
-}
-
-constexpr int kSplitChunk = 64;  // K per block when the product is split
-constexpr int kMaxSplit = 64;
-
-// Products with a small output and a long K (the weight gradients, K = the
-// batch) are split over K into kSplitChunk chunks reduced in fixed order;
-// `split` (kMaxSplit * 64 * 64 floats) holds the partials.
-template <bool TA, bool TB>
-vg_status gemm(int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
-               int ldc, hipStream_t s, float *split = nullptr) {
-    const dim3 tiles(vg::ceil_div(M, 64), vg::ceil_div(N, 64));
-    int nsplit = split && M <= 64 && N <= 64 ? (int)vg::ceil_div(K, kSplitChunk) : 1;
-    if (nsplit > kMaxSplit) nsplit = kMaxSplit;
-    if (nsplit <= 1)
-        return vg::launch("vg_mlp_gemm", k_gemm<TA, TB>, tiles, dim3(256), 0, s, M, N, K, A, lda, B,
-                          ldb, C, ldc, K);
-    const int kc = (int)(vg::ceil_div(vg::ceil_div(K, nsplit), 32) * 32);
-    nsplit = (int)vg::ceil_div(K, kc);
-    VG_TRY(vg::launch("vg_mlp_gemm", k_gemm<TA, TB>, dim3(tiles.x, tiles.y, nsplit), dim3(256), 0, s,
-                      M, N, K, A, lda, B, ldb, split, N, kc));
-    return vg::launch("vg_mlp_gemm_reduce", k_reduce_split, dim3(vg::ceil_div(M * N, 256)), dim3(256),
-                      0, s, (const float *)split, nsplit, M, N, N, C, ldc);
-}
-// C = A B, C = A^T B, C = A B^T
-vg_status gemm_nn(int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
-                  int ldc, hipStream_t s) {
-    return gemm<false, false>(M, N, K, A, lda, B, ldb, C, ldc, s);
-}
-vg_status gemm_tn(int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
-                  int ldc, hipStream_t s, float *split) {
-    return gemm<true, false>(M, N, K, A, lda, B, ldb, C, ldc, s, split);
-}
-vg_status gemm_nt(int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
-                  int ldc, hipStream_t s) {
-    return gemm<false, true>(M, N, K, A, lda, B, ldb, C, ldc, s);
-}
-
-// ------------------------------------------------------------------ elementwise
-__global__ void k_bias_gelu(float *__restrict__ Z, float *__restrict__ A,
-                            const float *__restrict__ b, size_t n, int cols) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float z = Z[i] + b[i % cols];
-    Z[i] = z;
-    A[i] = gelu(z);
-}
-
-__global__ void k_bias_add(float *__restrict__ Y, const float *__restrict__ b, size_t n, int cols) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    Y[i] += b[i % cols];
-}
-
-__global__ void k_gelu_back(float *__restrict__ dA, const float *__restrict__ Z, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    dA[i] *= gelu_grad(Z[i]);
-}
-
-// Loss of the correction vectors B c (B = identity when null) against T:
-// dY = 2 B^T (B c - T) / (3 rows) on the 3 live columns, 0 on the padding;
-// one block partial of sum |B c - T|^2 per block.
-__global__ __launch_bounds__(256) void k_loss_grad(const float *__restrict__ Y,
-                                                   const float *__restrict__ Bm,
-                                                   const float *__restrict__ T,
-                                                   float *__restrict__ dY, uint32_t rows,
-                                                   float scale, float *__restrict__ partial) {
-    __shared__ float red[256];
-    const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    float s = 0.f;
-    if (r < rows) {
-        const float *y = Y + (size_t)r * kOutPad;
-        float e[3], g[3];
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            float v = y[i];
-            if (Bm) {
-                const float *b = Bm + (size_t)r * 9 + 3 * i;
-                v = b[0] * y[0] + b[1] * y[1] + b[2] * y[2];
-            }
-            e[i] = v - T[(size_t)r * kOut + i];
-            s += e[i] * e[i];
-        }
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            g[k] = e[k];
-            if (Bm) {
-                const float *b = Bm + (size_t)r * 9;
-                g[k] = b[k] * e[0] + b[3 + k] * e[1] + b[6 + k] * e[2];
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < kOutPad; ++c) dY[(size_t)r * kOutPad + c] = c < kOut ? scale * g[c] : 0.f;
+    for (int v = 0; v < 4; ++v) {
+        o[kOffW1 + (g4 + v) * kHid + wave * 16 + r16] = gw1[0][0][v];
+        o[kOffW4 + (wave * 16 + g4 + v) * kOutPad + r16] = gw4[0][0][v];
     }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    // bias gradients: over the four row groups of a wave, then the two waves
+    // of a column
+    auto bias_out = [&](float(&gb)[2], int off) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            float t = gb[j];
+            t += __shfl_xor(t, 16);
+            t += __shfl_xor(t, 32);
+            if (lane < 16) L.bias_sum[wave & 1][wn + j * 16 + r16] = t;
+        }
         __syncthreads();
+        if (tid < kHid) o[off + tid] = L.bias_sum[0][tid] + L.bias_sum[1][tid];
+        __syncthreads();
+    };
+    bias_out(gb1, kOffB1);
+    bias_out(gb2, kOffB2);
+    bias_out(gb3, kOffB3);
+    if (wave == 0) {
+#pragma unroll
+        for (int w = 32; w; w >>= 1) {
+            loss += __shfl_xor(loss, w);
+#pragma unroll
+            for (int k = 0; k < kOut; ++k) gb4[k] += __shfl_xor(gb4[k], w);
+        }
+        if (lane < kOutPad)
+            o[kOffB4 + lane] = lane == 0 ? gb4[0] : lane == 1 ? gb4[1] : lane == 2 ? gb4[2] : 0.f;
+        if (lane == 0) o[kPadParams] = loss;
     }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-// Column sums of D [rows][cols] (cols divides 256) in a fixed order, in two
-// stages: workgroup b sums rows [b chunk, (b + 1) chunk) into part[b][cols],
-// then k_colsum_final adds the partials in workgroup order.
-constexpr uint32_t kColRows = 128;  // rows per workgroup unless the scratch needs more
-__global__ __launch_bounds__(256) void k_colsum_part(const float *__restrict__ D, uint32_t rows,
-                                                     int cols, uint32_t chunk,
-                                                     float *__restrict__ part) {
-    __shared__ float red[256];
-    const int t = threadIdx.x, c = t % cols, g = t / cols, ng = 256 / cols;
-    const uint32_t r0 = blockIdx.x * chunk;
-    const uint32_t r1 = rows - r0 < chunk ? rows : r0 + chunk;
+// Sums of the nslab slabs: 64 parameters per workgroup, each wave a run of
+// the slabs with its loads in flight together, the four runs added in order.
+// With ADAM the parameters are updated at once and only the loss is written.
+template <bool ADAM>
+__global__ __launch_bounds__(256) void k_mlp_sum(const float *__restrict__ part, uint32_t nslab,
+                                                 Adam opt, float *__restrict__ sum) {
+    __shared__ float red[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i = blockIdx.x * 64 + lane;
+    const uint32_t per = (nslab + 3) / 4, z0 = wave * per, z1 = min(nslab, z0 + per);
     float s = 0.f;
-    for (uint32_t r = r0 + (uint32_t)g; r < r1; r += (uint32_t)ng) s += D[(size_t)r * cols + c];
-    red[t] = s;
+    if (i < kSlab) {
+#pragma unroll 16
+        for (uint32_t z = z0; z < z1; ++z) s += part[(size_t)z * kSlab + i];
+    }
+    red[wave][lane] = s;
     __syncthreads();
-    if (t < cols) {
-        float a = 0.f;
-        for (int j = 0; j < ng; ++j) a += red[j * cols + t];
-        part[(size_t)blockIdx.x * cols + t] = a;
-    }
-}
-
-__global__ void k_colsum_final(const float *__restrict__ part, uint32_t nparts, int cols,
-                               float *__restrict__ out) {
-    const int t = threadIdx.x;
-    if (t >= cols) return;
-    float a = 0.f;
-    for (uint32_t b = 0; b < nparts; ++b) a += part[(size_t)b * cols + t];
-    out[t] = a;
-}
-
-// Column sums of D [rows][cols] into out, with `part` (kMaxSplit * 64 * 64
-// floats, the split products' scratch, free between products) holding the
-// per-workgroup partials.
-vg_status colsum(const float *D, uint32_t rows, int cols, float *out, float *part,
-                 hipStream_t s) {
-    VG_REQUIRE(cols > 0 && cols <= 64 && 256 % cols == 0, "column sum: cols must divide 256");
-    const size_t max_parts = (size_t)kMaxSplit * 64 * 64 / cols;
-    uint32_t chunk = kColRows;
-    if (vg::ceil_div(rows, chunk) > max_parts) chunk = vg::ceil_div(rows, max_parts);
-    const uint32_t nparts = vg::ceil_div(rows, chunk);
-    VG_TRY(vg::launch("vg_mlp_colsum", k_colsum_part, dim3(nparts), dim3(256), 0, s, D, rows, cols,
-                      chunk, part));
-    return vg::launch("vg_mlp_colsum", k_colsum_final, dim3(1), dim3(64), 0, s, (const float *)part,
-                      nparts, cols, out);
-}
-
-__global__ void k_sum_partials(const float *__restrict__ partial, uint32_t n, float *__restrict__ out) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        float s = 0.f;
-        for (uint32_t i = 0; i < n; ++i) s += partial[i];
-        out[0] = s;
-    }
-}
-
-__global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m1,
-                       float *__restrict__ m2, int n, float lr, float b1, float b2, float eps,
-                       float bc1, float bc2) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float a = b1 * m1[i] + (1.0f - b1) * gi;
-    const float v = b2 * m2[i] + (1.0f - b2) * gi * gi;
-    m1[i] = a;
-    m2[i] = v;
-    p[i] -= lr * (a / bc1) / (sqrtf(v / bc2) + eps);
-}
-
-__global__ void k_copy_cols(const float *__restrict__ src, int lds, float *__restrict__ dst, int ldd,
-                            int cols, uint32_t rows) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)rows * cols) return;
-    const size_t r = i / cols, c = i % cols;
-    dst[r * ldd + c] = src[r * lds + c];
+    if (wave || i >= kSlab) return;
+    s = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+    if (ADAM && i < kPadParams)
+        adam_update(opt, i, s);
+    else
+        sum[i] = s;
 }
 
 // ------------------------------------------------------------------ inference packing
@@ -876,7 +970,7 @@ __global__ __launch_bounds__(256) void k_mlp_samples(const vg::TreeView tv, vg_g
 
 // ------------------------------------------------------------------ handle
 struct vg_mlp {
-    float *params = nullptr, *grad = nullptr, *m1 = nullptr, *m2 = nullptr;
+    float *params = nullptr, *m1 = nullptr, *m2 = nullptr;
     __bf16 *packed = nullptr;
     bool packed_ok = false;
     uint32_t step = 0;
@@ -928,90 +1022,49 @@ vg_status ensure_packed(vg_mlp *m, hipStream_t s) {
     return VG_OK;
 }
 
-// Activations of one batch.
-struct Acts {
-    float *Z1, *A1, *Z2, *A2, *Z3, *A3, *Y, *dY, *dA, *partial, *loss, *split;
-    void *base = nullptr;
+template <bool GRAD>
+vg_status mlp_pass(const vg_mlp *m, const float *X, const float *Bm, const float *T, uint32_t rows,
+                   uint32_t blocks, float *out, hipStream_t s) {
+    const size_t bytes = GRAD ? sizeof(GradLds) : sizeof(FwdLds);
+    VG_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_mlp_pass<GRAD>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    return launch(GRAD ? "vg_mlp_gradients" : "vg_mlp_forward", k_mlp_pass<GRAD>, dim3(blocks),
+                  dim3(256), bytes, s, (const float *)m->params, X, Bm, T, rows,
+                  2.0f / (3.0f * (float)rows), out);
+}
+
+// Scratch of the gradients of one batch: a slab per workgroup and their sum.
+struct Grads {
+    float *slabs = nullptr, *sum = nullptr;
+    uint32_t blocks = 0;
 };
 
-vg_status acts_alloc(Acts *a, uint32_t rows, hipStream_t s) {
-    const size_t h = (size_t)rows * kHid, y = (size_t)rows * kOutPad;
-    const size_t nparts = ceil_div(rows, 256);
-    const size_t nsplit = (size_t)kMaxSplit * 64 * 64;
-    const size_t total = 7 * h + 2 * y + nparts + 1 + nsplit;
-    VG_TRY(salloc(&a->base, total * sizeof(float), s));
-    float *p = (float *)a->base;
-    a->Z1 = p; p += h; a->A1 = p; p += h; a->Z2 = p; p += h; a->A2 = p; p += h;
-    a->Z3 = p; p += h; a->A3 = p; p += h; a->dA = p; p += h;
-    a->Y = p; p += y; a->dY = p; p += y;
-    a->partial = p; p += nparts; a->loss = p; p += 1;
-    a->split = p;
+vg_status grads_alloc(Grads *a, uint32_t rows, hipStream_t s) {
+    a->blocks = std::min<uint32_t>(ceil_div(rows, kRows), kRowTiles);
+    VG_TRY(salloc((void **)&a->slabs, ((size_t)a->blocks + 1) * kSlab * sizeof(float), s));
+    a->sum = a->slabs + (size_t)a->blocks * kSlab;
     return VG_OK;
 }
 
-vg_status forward(vg_mlp *m, const float *X, uint32_t rows, Acts &a, hipStream_t s) {
-    const float *P = m->params;
-    const size_t h = (size_t)rows * kHid;
-    const dim3 eg(ceil_div(h, 256));
-    VG_TRY(gemm_nn(rows, kHid, kIn, X, kIn, P + kOffW1, kHid, a.Z1, kHid, s));
-    VG_TRY(launch("vg_mlp_gelu", k_bias_gelu, eg, dim3(256), 0, s, a.Z1, a.A1, P + kOffB1, h, kHid));
-    VG_TRY(gemm_nn(rows, kHid, kHid, a.A1, kHid, P + kOffW2, kHid, a.Z2, kHid, s));
-    VG_TRY(launch("vg_mlp_gelu", k_bias_gelu, eg, dim3(256), 0, s, a.Z2, a.A2, P + kOffB2, h, kHid));
-    VG_TRY(gemm_nn(rows, kHid, kHid, a.A2, kHid, P + kOffW3, kHid, a.Z3, kHid, s));
-    VG_TRY(launch("vg_mlp_gelu", k_bias_gelu, eg, dim3(256), 0, s, a.Z3, a.A3, P + kOffB3, h, kHid));
-    VG_TRY(gemm_nn(rows, kOutPad, kHid, a.A3, kHid, P + kOffW4, kOutPad, a.Y, kOutPad, s));
-    const size_t ny = (size_t)rows * kOutPad;
-    VG_TRY(launch("vg_mlp_bias", k_bias_add, dim3(ceil_div(ny, 256)), dim3(256), 0, s, a.Y,
-                  (const float *)(P + kOffB4), ny, kOutPad));
-    return VG_OK;
+// Gradients (padded layout) and summed squares of one batch into a.sum.
+vg_status gradients(const vg_mlp *m, const float *X, const float *Bm, const float *T, uint32_t rows,
+                    const Grads &a, hipStream_t s) {
+    VG_TRY(mlp_pass<true>(m, X, Bm, T, rows, a.blocks, a.slabs, s));
+    return launch("vg_mlp_sum", k_mlp_sum<false>, dim3(ceil_div(kSlab, 64)), dim3(256), 0, s,
+                  (const float *)a.slabs, a.blocks, Adam{}, a.sum);
 }
 
-// Loss gradient and parameter gradients into m->grad (padded layout).
-vg_status backward(vg_mlp *m, const float *X, const float *Bm, const float *T, uint32_t rows,
-                   Acts &a, hipStream_t s) {
-    const float *P = m->params;
-    float *G = m->grad;
-    const size_t h = (size_t)rows * kHid;
-    const dim3 eg(ceil_div(h, 256));
-    const uint32_t nparts = ceil_div(rows, 256);
-    VG_TRY(launch("vg_mlp_loss", k_loss_grad, dim3(nparts), dim3(256), 0, s, (const float *)a.Y, Bm,
-                  T, a.dY, rows, 2.0f / (3.0f * (float)rows), a.partial));
-    VG_TRY(launch("vg_mlp_loss", k_sum_partials, dim3(1), dim3(64), 0, s, (const float *)a.partial,
-                  nparts, a.loss));
-    // output layer
-    VG_TRY(gemm_tn(kHid, kOutPad, rows, a.A3, kHid, a.dY, kOutPad, G + kOffW4, kOutPad, s, a.split));
-    VG_TRY(colsum(a.dY, rows, kOutPad, G + kOffB4, a.split, s));
-    VG_TRY(gemm_nt(rows, kHid, kOutPad, a.dY, kOutPad, P + kOffW4, kOutPad, a.dA, kHid, s));
-    // hidden layers 3, 2, 1: dZ = dA * gelu'(Z), dW = A_prev^T dZ, dA_prev = dZ W^T
-    struct L { float *Z; const float *Aprev; int lda_prev, kprev, offW, offB; };
-    const L layers[3] = {{a.Z3, a.A2, kHid, kHid, kOffW3, kOffB3},
-                         {a.Z2, a.A1, kHid, kHid, kOffW2, kOffB2},
-                         {a.Z1, X, kIn, kIn, kOffW1, kOffB1}};
-    for (int li = 0; li < 3; ++li) {
-        const L &L_ = layers[li];
-        VG_TRY(launch("vg_mlp_gelu_back", k_gelu_back, eg, dim3(256), 0, s, a.dA,
-                      (const float *)L_.Z, h));
-        VG_TRY(gemm_tn(L_.kprev, kHid, rows, L_.Aprev, L_.lda_prev, a.dA, kHid,
-                       G + L_.offW, kHid, s, a.split));
-        VG_TRY(colsum(a.dA, rows, kHid, G + L_.offB, a.split, s));
-        if (li < 2) {
-            // dA_prev = dZ W^T, written over the previous layer's Z (its
-            // pre-activation is still needed: use A_prev's slot instead)
-            float *dprev = (li == 0) ? a.A3 : a.A2;  // A3/A2 are no longer needed
-            VG_TRY(gemm_nt(rows, kHid, kHid, a.dA, kHid, P + L_.offW, kHid, dprev, kHid, s));
-            VG_HIP(hipMemcpyAsync(a.dA, dprev, h * sizeof(float), hipMemcpyDeviceToDevice, s));
-        }
-    }
-    return VG_OK;
-}
-
-vg_status adam_step(vg_mlp *m, float lr, hipStream_t s) {
+// One Adam step on the batch; the summed squares go to a.sum[kPadParams].
+vg_status adam_step(vg_mlp *m, const float *X, const float *Bm, const float *T, uint32_t rows,
+                    float lr, const Grads &a, hipStream_t s) {
+    VG_TRY(mlp_pass<true>(m, X, Bm, T, rows, a.blocks, a.slabs, s));
     m->step += 1;
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float bc1 = 1.0f - std::pow(b1, (float)m->step), bc2 = 1.0f - std::pow(b2, (float)m->step);
+    Adam o{m->params, m->m1, m->m2, lr, 0.9f, 0.999f, 1e-8f, 0.f, 0.f};
+    o.bc1 = 1.0f - std::pow(o.b1, (float)m->step);
+    o.bc2 = 1.0f - std::pow(o.b2, (float)m->step);
     m->packed_ok = false;
-    return launch("vg_mlp_adam", k_adam, dim3(ceil_div(kPadParams, 256)), dim3(256), 0, s, m->params,
-                  (const float *)m->grad, m->m1, m->m2, kPadParams, lr, b1, b2, eps, bc1, bc2);
+    return launch("vg_mlp_sum", k_mlp_sum<true>, dim3(ceil_div(kSlab, 64)), dim3(256), 0, s,
+                  (const float *)a.slabs, a.blocks, o, a.sum);
 }
 
 vg_status layer_inv_h(const TreeView &tv, float *inv_h) {
@@ -1037,14 +1090,13 @@ VG_API vg_status vg_mlp_create(vg_mlp **out, uint64_t seed) {
         vg_mlp_destroy(m);
         return st;
     };
-    hipError_t e = hipMalloc((void **)&m->params, 4 * kPadParams * sizeof(float));
+    hipError_t e = hipMalloc((void **)&m->params, 3 * kPadParams * sizeof(float));
     if (e != hipSuccess) return fail(device_error(e, "hipMalloc mlp", __FILE__, __LINE__));
-    m->grad = m->params + kPadParams;
-    m->m1 = m->grad + kPadParams;
+    m->m1 = m->params + kPadParams;
     m->m2 = m->m1 + kPadParams;
     e = hipMalloc((void **)&m->packed, kPackedElems * sizeof(__bf16));
     if (e != hipSuccess) return fail(device_error(e, "hipMalloc mlp", __FILE__, __LINE__));
-    e = hipMemset(m->params, 0, 4 * kPadParams * sizeof(float));
+    e = hipMemset(m->params, 0, 3 * kPadParams * sizeof(float));
     if (e != hipSuccess) return fail(device_error(e, "hipMemset mlp", __FILE__, __LINE__));
     // uniform +-sqrt(6 / (fan_in + fan_out)) weights from splitmix64(seed),
     // zero biases
@@ -1101,13 +1153,21 @@ VG_API vg_status vg_mlp_forward(vg_mlp *m, const float *x, uint32_t n, float *y,
     if (n == 0) return VG_OK;
     VG_REQUIRE(x && y, "null buffer");
     hipStream_t s = (hipStream_t)stream;
-    Acts a;
-    VG_TRY(acts_alloc(&a, n, s));
-    vg_status st = forward(m, x, n, a, s);
-    if (st == VG_OK)
-        st = launch("vg_mlp_copy", k_copy_cols, dim3(ceil_div((size_t)n * kOut, 256)), dim3(256), 0,
-                    s, (const float *)a.Y, kOutPad, y, kOut, kOut, n);
-    sfree(a.base, s);
+    // a workgroup writes rows of y while others still read x: where the two
+    // overlap, y goes by way of scratch
+    const uintptr_t xa = (uintptr_t)x, ya = (uintptr_t)y;
+    const size_t xb = (size_t)n * kIn * sizeof(float), yb = (size_t)n * kOut * sizeof(float);
+    const uint32_t blocks = std::min<uint32_t>(ceil_div(n, kRows), 3 * kRowTiles);
+    if (ya >= xa + xb || xa >= ya + yb)
+        return mlp_pass<false>(m, x, nullptr, nullptr, n, blocks, y, s);
+    float *tmp = nullptr;
+    VG_TRY(salloc((void **)&tmp, yb, s));
+    vg_status st = mlp_pass<false>(m, x, nullptr, nullptr, n, blocks, tmp, s);
+    if (st == VG_OK) {
+        const hipError_t e = hipMemcpyAsync(y, tmp, yb, hipMemcpyDeviceToDevice, s);
+        if (e != hipSuccess) st = device_error(e, "mlp output copy", __FILE__, __LINE__);
+    }
+    sfree(tmp, s);
     return st;
 }
 
@@ -1116,23 +1176,19 @@ VG_API vg_status vg_mlp_gradients(vg_mlp *m, const float *x, const float *basis,
     VG_REQUIRE(m && x && t && grad, "null argument");
     VG_REQUIRE(n > 0, "empty batch");
     hipStream_t s = (hipStream_t)stream;
-    Acts a;
-    VG_TRY(acts_alloc(&a, n, s));
-    vg_status st = forward(m, x, n, a, s);
-    if (st == VG_OK) st = backward(m, x, basis, t, n, a, s);
-    float l = 0.f;
-    std::vector<float> g(kPadParams);
+    Grads a;
+    VG_TRY(grads_alloc(&a, n, s));
+    vg_status st = gradients(m, x, basis, t, n, a, s);
+    std::vector<float> g(kSlab);
     if (st == VG_OK) {
-        hipError_t e = hipMemcpyAsync(&l, a.loss, sizeof(float), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(g.data(), m->grad, kPadParams * sizeof(float), hipMemcpyDeviceToHost, s);
+        hipError_t e = hipMemcpyAsync(g.data(), a.sum, kSlab * sizeof(float), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) st = device_error(e, "mlp gradient copy", __FILE__, __LINE__);
     }
-    sfree(a.base, s);
+    sfree(a.slabs, s);
     if (st != VG_OK) return st;
     padded_to_compact(g, grad);
-    if (loss) *loss = l / (3.0f * (float)n);
+    if (loss) *loss = g[kPadParams] / (3.0f * (float)n);
     return VG_OK;
 }
 
@@ -1142,26 +1198,23 @@ VG_API vg_status vg_mlp_train(vg_mlp *m, const float *x, const float *basis, con
     VG_REQUIRE(m && x && t, "null argument");
     VG_REQUIRE(batch > 0 && batch <= n, "batch must be in [1, n]");
     hipStream_t s = (hipStream_t)stream;
-    Acts a;
-    VG_TRY(acts_alloc(&a, batch, s));
+    Grads a;
+    VG_TRY(grads_alloc(&a, batch, s));
     vg_status st = VG_OK;
     const uint64_t span = (uint64_t)n - batch + 1;
     for (uint32_t it = 0; it < steps && st == VG_OK; ++it) {
         const uint64_t off = ((uint64_t)it * batch) % span;
-        const float *xb = x + off * kIn, *tb = t + off * kOut;
         const float *bb = basis ? basis + off * 9 : nullptr;
-        st = forward(m, xb, batch, a, s);
-        if (st == VG_OK) st = backward(m, xb, bb, tb, batch, a, s);
-        if (st == VG_OK) st = adam_step(m, lr, s);
+        st = adam_step(m, x + off * kIn, bb, t + off * kOut, batch, lr, a, s);
     }
     float l = 0.f;
     if (st == VG_OK && final_loss) {
-        hipError_t e = hipMemcpyAsync(&l, a.loss, sizeof(float), hipMemcpyDeviceToHost, s);
+        hipError_t e = hipMemcpyAsync(&l, a.sum + kPadParams, sizeof(float), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) st = device_error(e, "mlp loss copy", __FILE__, __LINE__);
         *final_loss = l / (3.0f * (float)batch);
     }
-    sfree(a.base, s);
+    sfree(a.slabs, s);
     return st;
 }
 
