@@ -12,6 +12,7 @@
 //    against FP64 residuals (mixed-precision iterative refinement): an FP32
 //    field alone cannot reach a 1e-6 relative residual on large grids, since
 //    its rounding noise amplified by the Laplacian sits near 1e-4.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -208,16 +209,11 @@ __global__ void k_prolong_add(vg_grid_desc hi, float *__restrict__ uhi, vg_grid_
     for (int k = 0; k < 3; ++k) uhi[3 * o + k] += acc[k];
 }
 
-// FP64 coarsest solve: one workgroup, red-black Gauss-Seidel in double, on
-// a copy of u in LDS (IN_LDS, grids up to kCoarseLdsPoints) or in `work`.
-constexpr uint32_t kCoarseLdsPoints = 2048;  // 48 KB of doubles
-
-template <bool IN_LDS>
+// FP64 coarsest solve of grids too large for k_vcycle_lds: one workgroup,
+// red-black Gauss-Seidel in double on a copy of u in `w`.
 __global__ __launch_bounds__(256) void k_coarse_f64(vg_grid_desc g, float *__restrict__ u,
                                                     const float *__restrict__ f, int sweeps,
-                                                    double *__restrict__ work) {
-    __shared__ double lds[IN_LDS ? 3 * kCoarseLdsPoints : 1];
-    double *w = IN_LDS ? lds : work;
+                                                    double *__restrict__ w) {
     const uint32_t nx = g.np[0], nxy = nx * g.np[1], n = nxy * g.np[2];
     const double rx = 1.0 / g.cell[0], ry = 1.0 / g.cell[1], rz = 1.0 / g.cell[2];
     const double r2x = rx * rx, r2y = ry * ry, r2z = rz * rz;
@@ -232,42 +228,217 @@ __global__ __launch_bounds__(256) void k_coarse_f64(vg_grid_desc g, float *__res
             w[3 * o + k] = (s - (double)f[3 * o + k]) * inv;
         }
     };
-    if (n <= 64) {
-        // one point per lane of the first wave, colours ordered by wave
-        // barriers (a wave's LDS operations complete in order) instead of
-        // workgroup barriers
-        if (threadIdx.x < 64) {
-            const uint32_t o = threadIdx.x;
-            bool inner = false;
-            uint32_t parity = 0;
-            if (o < n) {
+    for (int it = 0; it < sweeps; ++it) {
+        for (uint32_t color = 0; color < 2; ++color) {
+            for (uint32_t o = threadIdx.x; o < n; o += blockDim.x) {
                 const Pt p = split(o, g.np[0], g.np[1]);
-                inner = !on_boundary(p, g);
-                parity = (p.x + p.y + p.z) & 1u;
+                if (on_boundary(p, g) || ((p.x + p.y + p.z) & 1u) != color) continue;
+                update(o);
             }
-            for (int it = 0; it < sweeps; ++it) {
-                for (uint32_t color = 0; color < 2; ++color) {
-                    if (inner && parity == color) update(o);
+            __syncthreads();
+        }
+    }
+    for (uint32_t i = threadIdx.x; i < 3 * n; i += blockDim.x) u[i] = (float)w[i];
+}
+
+// ------------------------------------------------------------------ coarse levels
+// The V-cycle's levels that fit a CU's LDS together, in one launch: the three
+// components decouple, so one workgroup each takes its component of f down
+// from the first of them to the coarsest and back.  The steps are those of
+// vcycle(): nu red-black sweeps, the residual, its full weighting, the
+// correction, nu sweeps; FP64 sweeps on the coarsest.  These levels hold at
+// most ten thousand points, so their sweeps are all latency: a launch of a
+// few microseconds each against a barrier.  (129x129x257, whose last four
+// levels from 17x17x33 on fit: 34 launches per cycle down to one, their kernels
+// 107 -> 39 us, a solve of six cycles 3.98 -> 3.61 ms.)
+constexpr size_t kLdsBytes = 160 * 1024;  // of a CU
+constexpr int kLdsThreads = 1024;
+
+struct LdsLevel {
+    int nx, ny, nz;
+    int u, f;              // float offsets of the level's fields in LDS
+    int shift;             // 2^shift >= one colour's points of an x row
+    int step_y, step_z;    // rows between a thread's visits, as (y, z)
+    Lap c;
+};
+struct LdsCycle {
+    LdsLevel lv[kMaxLayers];
+    int levels, work;      // float offset of the residual, or the coarsest's doubles
+    int nu, sweeps;        // smoothing sweeps; coarsest sweeps
+    float cell[3];         // of the coarsest
+};
+
+// op(o, ix, iy, iz) for this thread's interior points of one colour.
+template <typename Op>
+__device__ __forceinline__ void lds_color(const LdsLevel &v, int color, Op op) {
+    const int tx = (int)threadIdx.x & ((1 << v.shift) - 1), row = (int)threadIdx.x >> v.shift;
+    int z = row / (v.ny - 2), y = row - z * (v.ny - 2);
+    while (z < v.nz - 2) {
+        const int iy = y + 1, iz = z + 1;
+        const int ix = 1 + ((iy + iz + 1 + color) & 1) + 2 * tx;
+        if (ix <= v.nx - 2) op(ix + v.nx * (iy + v.ny * iz), ix, iy, iz);
+        y += v.step_y;
+        z += v.step_z;
+        if (y >= v.ny - 2) {
+            y -= v.ny - 2;
+            ++z;
+        }
+    }
+}
+template <typename Op>
+__device__ __forceinline__ void lds_interior(const LdsLevel &v, Op op) {
+    lds_color(v, 0, op);
+    lds_color(v, 1, op);
+}
+
+__device__ __forceinline__ void lds_smooth(const LdsLevel &v, float *lds, int sweeps) {
+    float *u = lds + v.u;
+    const float *f = lds + v.f;
+    const int sy = v.nx, sz = v.nx * v.ny;
+    for (int it = 0; it < 2 * sweeps; ++it) {
+        lds_color(v, it & 1, [&](int o, int, int, int) {
+#pragma clang fp contract(off)
+            const float s = (u[o + 1] + u[o - 1]) * v.c.r2x + (u[o + sy] + u[o - sy]) * v.c.r2y +
+                            (u[o + sz] + u[o - sz]) * v.c.r2z;
+            u[o] = (s - f[o]) * v.c.inv;
+        });
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(kLdsThreads) void k_vcycle_lds(LdsCycle C, float *__restrict__ u0,
+                                                            const float *__restrict__ f0) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int comp = (int)blockIdx.x, tid = (int)threadIdx.x;
+    const int n0 = C.lv[0].nx * C.lv[0].ny * C.lv[0].nz;
+#pragma unroll 4
+    for (int i = tid; i < n0; i += kLdsThreads) lds[C.lv[0].f + i] = f0[3 * (size_t)i + comp];
+    for (int i = tid; i < n0; i += kLdsThreads) lds[C.lv[0].u + i] = 0.f;
+    __syncthreads();
+
+    for (int l = 0; l + 1 < C.levels; ++l) {
+        const LdsLevel &v = C.lv[l], &w = C.lv[l + 1];
+        lds_smooth(v, lds, C.nu);
+        const float *u = lds + v.u, *f = lds + v.f;
+        float *r = lds + C.work;
+        const int sy = v.nx, sz = v.nx * v.ny;
+        lds_interior(v, [&](int o, int, int, int) {
+            const float lap = (u[o + 1] + u[o - 1]) * v.c.r2x + (u[o + sy] + u[o - sy]) * v.c.r2y +
+                              (u[o + sz] + u[o - sz]) * v.c.r2z - v.c.diag * u[o];
+            r[o] = f[o] - lap;
+        });
+        const int nw = w.nx * w.ny * w.nz;
+        for (int i = tid; i < nw; i += kLdsThreads) lds[w.u + i] = 0.f;
+        __syncthreads();
+        lds_interior(w, [&](int o, int ix, int iy, int iz) {
+            const float *h = r + 2 * ix + sy * (2 * iy) + sz * (2 * iz);
+            float acc = 0.f;
+#pragma unroll
+            for (int dz = -1; dz <= 1; ++dz)
+#pragma unroll
+                for (int dy = -1; dy <= 1; ++dy)
+#pragma unroll
+                    for (int dx = -1; dx <= 1; ++dx) {
+                        const int md = (dx != 0) + (dy != 0) + (dz != 0);
+                        acc += (float)(8 >> md) * h[dx + dy * sy + dz * sz];
+                    }
+            lds[w.f + o] = acc * (1.0f / 64.0f);
+        });
+        __syncthreads();
+    }
+
+    {  // coarsest, from zero, in double
+        const LdsLevel &v = C.lv[C.levels - 1];
+        double *w = (double *)(lds + C.work);
+        const float *f = lds + v.f;
+        const int sy = v.nx, sz = v.nx * v.ny, n = sz * v.nz;
+        const double rx = 1.0 / C.cell[0], ry = 1.0 / C.cell[1], rz = 1.0 / C.cell[2];
+        const double r2x = rx * rx, r2y = ry * ry, r2z = rz * rz;
+        const double inv = 1.0 / (2.0 * (r2x + r2y + r2z));
+        for (int i = tid; i < n; i += kLdsThreads) w[i] = 0.0;
+        __syncthreads();
+        auto update = [&](int o, int, int, int) {
+            const double s = (w[o + 1] + w[o - 1]) * r2x + (w[o + sy] + w[o - sy]) * r2y +
+                             (w[o + sz] + w[o - sz]) * r2z;
+            w[o] = (s - (double)f[o]) * inv;
+        };
+        if (n <= 64) {
+            // one point per lane of the first wave, colours ordered by wave
+            // barriers (a wave's LDS operations complete in order) instead of
+            // workgroup barriers
+            if (tid < 64) {
+                const Pt p = split((uint32_t)(tid < n ? tid : 0), (uint32_t)v.nx, (uint32_t)v.ny);
+                const bool inner = tid < n && p.x > 0 && p.y > 0 && p.z > 0 &&
+                                   (int)p.x < v.nx - 1 && (int)p.y < v.ny - 1 && (int)p.z < v.nz - 1;
+                const uint32_t parity = (p.x + p.y + p.z) & 1u;
+                for (int it = 0; it < 2 * C.sweeps; ++it) {
+                    if (inner && parity == (uint32_t)(it & 1)) update(tid, 0, 0, 0);
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                     __builtin_amdgcn_wave_barrier();
                     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                 }
             }
-        }
-        __syncthreads();
-    } else {
-        for (int it = 0; it < sweeps; ++it) {
-            for (uint32_t color = 0; color < 2; ++color) {
-                for (uint32_t o = threadIdx.x; o < n; o += blockDim.x) {
-                    const Pt p = split(o, g.np[0], g.np[1]);
-                    if (on_boundary(p, g) || ((p.x + p.y + p.z) & 1u) != color) continue;
-                    update(o);
-                }
+            __syncthreads();
+        } else {
+            for (int it = 0; it < 2 * C.sweeps; ++it) {
+                lds_color(v, it & 1, update);
                 __syncthreads();
             }
         }
+        for (int i = tid; i < n; i += kLdsThreads) lds[v.u + i] = (float)w[i];
+        __syncthreads();
     }
-    for (uint32_t i = threadIdx.x; i < 3 * n; i += blockDim.x) u[i] = (float)w[i];
+
+    for (int l = C.levels - 2; l >= 0; --l) {
+        const LdsLevel &v = C.lv[l], &w = C.lv[l + 1];
+        float *u = lds + v.u;
+        const float *c = lds + w.u;
+        const int cy = w.nx, cz = w.nx * w.ny;
+        lds_interior(v, [&](int o, int ix, int iy, int iz) {
+            // trilinear: the coarse points on either side, one where they coincide
+            const int bx = ix & 1, by = iy & 1, bz = iz & 1;
+            const int q = ix / 2 + cy * (iy / 2) + cz * (iz / 2);
+            const float x00 = c[q] + c[q + bx], x10 = c[q + by * cy] + c[q + by * cy + bx];
+            const int p = q + bz * cz;
+            const float x01 = c[p] + c[p + bx], x11 = c[p + by * cy] + c[p + by * cy + bx];
+            u[o] += 0.125f * ((x00 + x10) + (x01 + x11));
+        });
+        __syncthreads();
+        lds_smooth(v, lds, C.nu);
+    }
+    for (int i = tid; i < n0; i += kLdsThreads) u0[3 * (size_t)i + comp] = lds[C.lv[0].u + i];
+}
+
+// LDS bytes of k_vcycle_lds for levels l .. depth - 1, and its arguments: the
+// fields of every level, then the first level's residual or the coarsest's
+// doubles.
+size_t lds_cycle(const vg_grid_desc *levels, uint32_t l, uint32_t depth, LdsCycle *C) {
+    size_t at = 0, work = 0;
+    for (uint32_t i = l; i < depth; ++i) {
+        const vg_grid_desc &g = levels[i];
+        const size_t cap = capacity(g);
+        if (at + 2 * cap > kLdsBytes / sizeof(float)) return kLdsBytes + 1;
+        LdsLevel &v = C->lv[i - l];
+        v.nx = (int)g.np[0];
+        v.ny = (int)g.np[1];
+        v.nz = (int)g.np[2];
+        v.u = (int)at;
+        v.f = (int)(at + cap);
+        at += 2 * cap;
+        work = std::max(work, i + 1 < depth ? cap : 2 * cap);
+        v.shift = 0;
+        while ((1 << v.shift) < (v.nx - 1) / 2) ++v.shift;
+        if ((1 << v.shift) > kLdsThreads) return kLdsBytes + 1;
+        const int rows = kLdsThreads >> v.shift;
+        v.step_y = rows % (v.ny - 2);
+        v.step_z = rows / (v.ny - 2);
+        v.c = lap_coef(g);
+    }
+    at = (at + 1) & ~(size_t)1;
+    C->work = (int)at;
+    C->levels = (int)(depth - l);
+    for (int a = 0; a < 3; ++a) C->cell[a] = levels[depth - 1].cell[a];
+    return (at + work) * sizeof(float);
 }
 
 // FP64 residual of the compensated solution (hi + lo): writes the FP32
@@ -455,29 +626,37 @@ vg_status smooth(const vg_grid_desc &g, float *u, float *tmp, const float *f, in
 vg_status vcycle(vg_multigrid *m, uint32_t l, hipStream_t s) {
     const vg_grid_desc &g = m->vg[l];
     const size_t cap = capacity(g);
-    if (l + 1 == m->vdepth) {
-        const bool in_lds = cap <= kCoarseLdsPoints;
-        double *work = nullptr;
-        if (!in_lds) VG_TRY(salloc((void **)&work, 3 * cap * sizeof(double), s));
-        uint32_t dmax = g.np[0];
-        if (g.np[1] > dmax) dmax = g.np[1];
-        if (g.np[2] > dmax) dmax = g.np[2];
+    const int nu = 2;
+    auto coarse_sweeps = [&]() {
+        const uint32_t *np = m->vg[m->vdepth - 1].np;
+        const uint32_t dmax = std::max(std::max(np[0], np[1]), np[2]);
         // red-black Gauss-Seidel shrinks the slowest error mode by about
         // 1 - (pi / (dmax - 1))^2 per sweep, so dmax^2 + 16 sweeps leave
         // below 1e-4 of it for every coarsest size the hierarchy allows
         // (dmax <= 33): more than one V-cycle needs
-        int sweeps = (int)(dmax * dmax + 16);
-        if (sweeps > 20000) sweeps = 20000;
-        vg_status st =
-            in_lds ? launch("vg_mg_coarse_f64", k_coarse_f64<true>, dim3(1), dim3(256), 0, s, g,
-                            m->u[l], (const float *)m->f[l], sweeps, work)
-                   : launch("vg_mg_coarse_f64", k_coarse_f64<false>, dim3(1), dim3(256), 0, s, g,
-                            m->u[l], (const float *)m->f[l], sweeps, work);
-        if (work) sfree(work, s);
+        return (int)std::min<uint32_t>(dmax * dmax + 16, 20000);
+    };
+    // the levels that fit LDS from here on: in one launch (u[l] is zero, by
+    // the restriction or the two-sum)
+    LdsCycle C;
+    const size_t lds = lds_cycle(m->vg, l, m->vdepth, &C);
+    if (lds <= kLdsBytes) {
+        C.nu = nu;
+        C.sweeps = coarse_sweeps();
+        VG_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_vcycle_lds),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
+        return launch("vg_mg_coarse", k_vcycle_lds, dim3(3), dim3(kLdsThreads), lds, s, C, m->u[l],
+                      (const float *)m->f[l]);
+    }
+    if (l + 1 == m->vdepth) {
+        double *work = nullptr;
+        VG_TRY(salloc((void **)&work, 3 * cap * sizeof(double), s));
+        const vg_status st = launch("vg_mg_coarse_f64", k_coarse_f64, dim3(1), dim3(256), 0, s, g,
+                                    m->u[l], (const float *)m->f[l], coarse_sweeps(), work);
+        sfree(work, s);
         return st;
     }
-    const int nu1 = 2, nu2 = 2;
-    VG_TRY(smooth(g, m->u[l], m->r[l], m->f[l], nu1, s));
+    VG_TRY(smooth(g, m->u[l], m->r[l], m->f[l], nu, s));
     VG_TRY(launch("vg_mg_residual", k_residual32, dim3(ceil_div(cap, 256)), dim3(256), 0, s, g,
                   (const float *)m->u[l], (const float *)m->f[l], m->r[l], lap_coef(g)));
     const vg_grid_desc &gc = m->vg[l + 1];
@@ -487,7 +666,7 @@ vg_status vcycle(vg_multigrid *m, uint32_t l, hipStream_t s) {
     VG_TRY(vcycle(m, l + 1, s));
     VG_TRY(launch("vg_mg_prolong_add", k_prolong_add, dim3(ceil_div(cap, 256)), dim3(256), 0, s, g,
                   m->u[l], gc, (const float *)m->u[l + 1]));
-    return smooth(g, m->u[l], m->r[l], m->f[l], nu2, s);
+    return smooth(g, m->u[l], m->r[l], m->f[l], nu, s);
 }
 
 }  // namespace
