@@ -326,13 +326,13 @@ __device__ __forceinline__ void parent_add_moment(ParentSums &a, float4 p, float
 // not be written (k_leaf skip_empty).
 __device__ __forceinline__ void aggregate_point(const vg_grid_desc &gp, const vg_grid_desc &gc,
                                                 uint32_t dx, uint32_t dy, uint32_t dz, size_t o,
-                                                const float4 *__restrict__ Pc,
-                                                const float4 *__restrict__ Wc,
-                                                const float4 *__restrict__ Mc,
-                                                const uint32_t *__restrict__ cc,
-                                                float4 *__restrict__ Pp, float4 *__restrict__ Wp,
-                                                float4 *__restrict__ Mp,
-                                                uint32_t *__restrict__ Cp) {
+                                                const float4 *Pc,
+                                                const float4 *Wc,
+                                                const float4 *Mc,
+                                                const uint32_t *cc,
+                                                float4 *Pp, float4 *Wp,
+                                                float4 *Mp,
+                                                uint32_t *Cp) {
 #pragma clang fp contract(off)
     const uint32_t ix = (uint32_t)(o % gp.np[0]);
     const uint32_t iy = (uint32_t)((o / gp.np[0]) % gp.np[1]);
@@ -434,6 +434,32 @@ __global__ void k_aggregate_views(const TreeView *__restrict__ views, uint32_t l
     aggregate_point(gp, tv.layer[l - 1], tv.dec[l][0], tv.dec[l][1], tv.dec[l][2], o, Pc + tc,
                     Wc + tc, Mc + 3 * tc, cc ? cc + tc : nullptr, Pp + tp, Wp + tp, Mp + 3 * tp,
                     Cp + tp);
+}
+
+// One tree's layers of at most kTopPoints points, in one workgroup with a
+// barrier between layers: each is a single trip of it, all latency, and as
+// launches of one stream they took 5 us each (a tree of 4,096 vortons, whose
+// layers from 9x9x9 up are four launches: a frame 366 -> 355 us).  Batched
+// trees keep a launch per layer: those are replayed from a graph, where the
+// chain in one workgroup gained nothing on one tree of 65,536 vortons (176.6
+// against 178.3 us a frame) and lost on 256 trees (3.45 against 3.59 ms).
+constexpr size_t kTopPoints = 1024;
+struct TopLayers {
+    Nested ng;
+    uint32_t first;  // lowest layer formed here
+    float4 *P[kMaxLayers], *W[kMaxLayers], *M[kMaxLayers];
+    uint32_t *C[kMaxLayers];
+};
+__global__ __launch_bounds__(kTopPoints) void k_aggregate_top(TopLayers a) {
+    for (uint32_t l = a.first; l < a.ng.depth; ++l) {
+        const vg_grid_desc &gp = a.ng.layer[l];
+        const uint32_t *dec = a.ng.dec[l];
+        const size_t o = threadIdx.x;  // a layer never has more points than its children's
+        if (o < capacity(gp))
+            aggregate_point(gp, a.ng.layer[l - 1], dec[0], dec[1], dec[2], o, a.P[l - 1],
+                            a.W[l - 1], a.M[l - 1], nullptr, a.P[l], a.W[l], a.M[l], a.C[l]);
+        __syncthreads();
+    }
 }
 
 template <typename T>
@@ -1297,13 +1323,28 @@ VG_API vg_status vg_tree_build(vg_tree *t, const vg_grid_desc *tmpl, const vg_vo
                   (const uint32_t *)t->cell_start, (const uint32_t *)t->cell_count,
                   (const float4 *)t->sorted_p, (const float4 *)t->sorted_w, cap0, t->P[0],
                   t->W[0], t->M[0], (const TreeView *)nullptr, 0));
-    for (uint32_t l = 1; l < t->ng.depth; ++l) {
+    uint32_t top = 1;
+    while (top < t->ng.depth && capacity(t->ng.layer[top]) > kTopPoints) ++top;
+    if (top + 2 > t->ng.depth) top = t->ng.depth;  // less than two layers: a launch each
+    for (uint32_t l = 1; l < top; ++l) {
         const size_t cap = capacity(t->ng.layer[l]);
         VG_TRY(launch("vg_tree_aggregate", k_aggregate, dim3(ceil_div(cap, 256)), dim3(256), 0, s,
                       t->ng.layer[l], t->ng.layer[l - 1], t->ng.dec[l][0], t->ng.dec[l][1],
                       t->ng.dec[l][2], (const float4 *)t->P[l - 1], (const float4 *)t->W[l - 1],
                       (const float4 *)t->M[l - 1], (const uint32_t *)nullptr, t->P[l], t->W[l],
                       t->M[l], t->C[l]));
+    }
+    if (top < t->ng.depth) {
+        TopLayers a;
+        a.ng = t->ng;
+        a.first = top;
+        for (uint32_t l = 0; l < kMaxLayers; ++l) {
+            a.P[l] = t->P[l];
+            a.W[l] = t->W[l];
+            a.M[l] = t->M[l];
+            a.C[l] = t->C[l];
+        }
+        VG_TRY(launch("vg_tree_aggregate", k_aggregate_top, dim3(1), dim3(kTopPoints), 0, s, a));
     }
     t->built = true;
     return VG_OK;
