@@ -694,34 +694,59 @@ static SorPlan sor_plan_kept(const vg_grid_desc &g, uint32_t total, bool scratch
     return k.plan;
 }
 
-// Exposed to the multigrid driver.  scratch: 9 floats per point, or null for
-// an allocation on the stream.
+static bool sor_whole(const vg_grid_desc &g, const SorPlan &plan, uint32_t total) {
+    return plan.by > 0 && plan.passes == (int)total && plan.by == (int)g.np[1] - 2 &&
+           plan.bz == (int)g.np[2] - 2;
+}
+
+// The plan of a solve; scratch: whether it may read any.
+static SorPlan sor_plan_of(const vg_grid_desc &g, uint32_t steps, bool scratch) {
+    if (g.np[0] < 3 || g.np[1] < 3 || g.np[2] < 3 || steps == 0) return SorPlan();
+    // (an odd row stride and 32-bit offsets: see k_sor_block)
+    const bool fits =
+        (g.np[0] & 1u) && steps < (1u << 24) && 3 * capacity(g) < (size_t(1) << 31);
+    return fits ? sor_plan_kept(g, 2 * steps, scratch) : SorPlan();
+}
+
+// Floats of scratch that sor_solve reads if it is given them.
+size_t sor_scratch(const vg_grid_desc &g, uint32_t steps) {
+    const SorPlan plan = sor_plan_of(g, steps, true);
+    return plan.by > 0 && !sor_whole(g, plan, 2 * steps) ? 9 * capacity(g) : 0;
+}
+
+// No allocation may be made on the stream: it is being captured (or the
+// answer is not to be had).
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+    if (hipStreamIsCapturing(s, &capture) == hipSuccess)
+        return capture != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
+// Exposed to the multigrid driver.  scratch: `scratch_floats` of them, which
+// are used where they are the sor_scratch of the grid; without, an allocation
+// on the stream.
 vg_status sor_solve(const vg_grid_desc &g, float *soln, const float *lap, uint32_t steps,
-                    hipStream_t s, float *scratch) {
+                    hipStream_t s, float *scratch, size_t scratch_floats) {
     if (g.np[0] < 3 || g.np[1] < 3 || g.np[2] < 3) return VG_OK;  // no interior
     if (steps == 0) return VG_OK;
     const SorCoef c = sor_coef(g);
     const size_t n = capacity(g);
-    // a stream under capture takes no allocation: without scratch, its grids
-    // that do not fit one workgroup keep the row kernels
-    bool may = scratch != nullptr;
-    if (!scratch) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
-        if (hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
-        else may = capture == hipStreamCaptureStatusNone;
-    }
-    // (an odd row stride and 32-bit offsets: see k_sor_block)
-    const bool fits = (g.np[0] & 1u) && steps < (1u << 24) && 3 * n < (size_t(1) << 31);
-    const SorPlan plan = fits ? sor_plan_kept(g, 2 * steps, may) : SorPlan();
-    const bool whole = plan.by > 0 && plan.passes == (int)(2 * steps) &&
-                       plan.by == (int)g.np[1] - 2 && plan.bz == (int)g.np[2] - 2;
+    if (scratch_floats < 9 * n) scratch = nullptr;
+    SorPlan plan = sor_plan_of(g, steps, scratch || !capturing(s));
+    bool whole = sor_whole(g, plan, 2 * steps);
     float *own = nullptr;
     if (plan.by > 0 && !whole && !scratch) {
-        // (no memory for it: the row kernels need none)
-        if (salloc((void **)&own, 9 * n * sizeof(float), s) == VG_OK) scratch = own;
-        else (void)hipGetLastError();
+        if (salloc((void **)&own, 9 * n * sizeof(float), s) == VG_OK) {
+            scratch = own;
+        } else {  // no memory for it: the solve that needs none
+            (void)hipGetLastError();
+            plan = sor_plan_of(g, steps, false);
+            whole = sor_whole(g, plan, 2 * steps);
+        }
     }
-    if (plan.by > 0 && (whole || scratch)) {
+    if (plan.by > 0) {
         VG_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_sor_block),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSorLdsBytes));
         SorBlock b;
@@ -881,7 +906,7 @@ VG_API vg_status vg_sor_solve(const vg_grid_desc *g, float *soln, const float *l
         if (g->np[2] > m) m = g->np[2];
         n = 2 * m;
     }
-    return sor_solve(*g, soln, lap, n, (hipStream_t)s, nullptr);
+    return sor_solve(*g, soln, lap, n, (hipStream_t)s, nullptr, 0);
 }
 
 VG_API vg_status vg_curl(const vg_grid_desc *g, const float *a, float *out, vg_stream s) {

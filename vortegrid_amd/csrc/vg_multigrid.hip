@@ -21,7 +21,9 @@
 
 namespace vg {
 vg_status sor_solve(const vg_grid_desc &g, float *soln, const float *lap, uint32_t steps,
-                    hipStream_t s, float *scratch);
+                    hipStream_t s, float *scratch, size_t scratch_floats);
+size_t sor_scratch(const vg_grid_desc &g, uint32_t steps);
+bool capturing(hipStream_t s);
 vg_status inject(const vg_grid_desc &lo, float *lf, const vg_grid_desc &hi, const float *hf,
                  hipStream_t s);
 vg_status prolong_interior(const vg_grid_desc &hi, float *hf, const vg_grid_desc &lo,
@@ -35,7 +37,7 @@ struct vg_multigrid {
     float *W[vg::kMaxLayers] = {};
     size_t cap[vg::kMaxLayers] = {};
     uint32_t cascade_layers = 0;  // layers holding values after the last cascade
-    float *sor = nullptr;         // the smoother's scratch, 9 floats per finest point
+    float *sor = nullptr;         // the smoother's scratch, where a layer's solve reads any
     size_t sor_cap = 0;
     // V-cycle hierarchy
     uint32_t vdepth = 0;
@@ -709,8 +711,12 @@ VG_API vg_status vg_mg_cascade(vg_multigrid *m, const vg_grid_desc *g, float *a0
         VG_TRY(grow(&m->W[l], &c2, 3 * capacity(ng.layer[l])));
         m->cap[l] = c1 < c2 ? c1 : c2;
     }
-    // (without it the smoother takes its row kernels)
-    if (grow(&m->sor, &m->sor_cap, 9 * capacity(ng.layer[0])) != VG_OK) (void)hipGetLastError();
+    size_t sor = 0;
+    for (uint32_t l = 0; l < ng.depth; ++l) sor = std::max(sor, sor_scratch(ng.layer[l], steps));
+    // (what is there serves the layers that it is enough for, the others do
+    // without: under capture, and where there is no memory for more)
+    if (sor > m->sor_cap && !capturing(s) && grow(&m->sor, &m->sor_cap, sor) != VG_OK)
+        (void)hipGetLastError();
     float *A[kMaxLayers];
     const float *W[kMaxLayers];
     A[0] = a0;
@@ -722,7 +728,7 @@ VG_API vg_status vg_mg_cascade(vg_multigrid *m, const vg_grid_desc *g, float *a0
     // Cold start: interior of the finest layer is zero (vortonSim.cpp:2531).
     VG_TRY(launch("vg_mg_zero_interior", k_zero_interior, dim3(ceil_div(capacity(*g), 256)),
                   dim3(256), 0, s, *g, a0));
-    VG_TRY(sor_solve(ng.layer[0], A[0], W[0], steps, s, m->sor));
+    VG_TRY(sor_solve(ng.layer[0], A[0], W[0], steps, s, m->sor, m->sor_cap));
     uint32_t max_valid = 0;
     for (uint32_t l = 1; l < ng.depth; ++l) {
         const uint32_t *np = ng.layer[l].np;
@@ -732,7 +738,7 @@ VG_API vg_status vg_mg_cascade(vg_multigrid *m, const vg_grid_desc *g, float *a0
         if (md > 2) {
             VG_TRY(inject(ng.layer[l], m->W[l], ng.layer[l - 1], W[l - 1], s));
             VG_TRY(inject(ng.layer[l], A[l], ng.layer[l - 1], A[l - 1], s));
-            VG_TRY(sor_solve(ng.layer[l], A[l], W[l], steps, s, m->sor));
+            VG_TRY(sor_solve(ng.layer[l], A[l], W[l], steps, s, m->sor, m->sor_cap));
         } else {
             max_valid = l - 1;
             break;
@@ -740,7 +746,7 @@ VG_API vg_status vg_mg_cascade(vg_multigrid *m, const vg_grid_desc *g, float *a0
     }
     for (uint32_t l = max_valid; l >= 1; --l) {
         VG_TRY(prolong_interior(ng.layer[l - 1], A[l - 1], ng.layer[l], A[l], s));
-        VG_TRY(sor_solve(ng.layer[l - 1], A[l - 1], W[l - 1], steps, s, m->sor));
+        VG_TRY(sor_solve(ng.layer[l - 1], A[l - 1], W[l - 1], steps, s, m->sor, m->sor_cap));
     }
     m->cascade_layers = max_valid + 1;
     return VG_OK;
