@@ -613,71 +613,155 @@ vg_status zero_fill(void *p, size_t bytes, hipStream_t s) {
 }
 
 // How `passes` colour passes over a grid are dealt to k_sor_block launches;
-// by == 0: they are not (rows too long for the LDS).
+// by == 0: they are not (rows too long for the LDS, or the row kernels faster).
 struct SorPlan {
     int by = 0, bz = 0, passes = 0, slots = 0, slot_threads = 0, threads = 0;
+    int rounds = 0;   // of workgroups on the chip
     size_t lds = 0;
     double us = 0.0;  // estimated time of all passes
 };
+// What a plan may read besides the grid: nothing, an allocation of its own on
+// the stream, one of the size that the thread's last solve asked for, or
+// scratch that is there.
+enum class SorScratch { None, Own, Again, Given };
+
+static bool sor_whole(const vg_grid_desc &g, const SorPlan &plan, uint32_t total) {
+    return plan.by > 0 && plan.passes == (int)total && plan.by == (int)g.np[1] - 2 &&
+           plan.bz == (int)g.np[2] - 2;
+}
 
 // Chooses among a grid's plans by an estimate of their time from what was
 // measured: 3 us to start a launch, staging and writing back at 14 bytes a
 // nanosecond, and per tick kSorChunk steps of 160 cycles, or 85 per wave
 // that shares its SIMD, and 400 for the barrier and the chunk's first reads.
 // Workgroups beyond what the 256 CUs hold at once follow in rounds.
-static SorPlan sor_plan(const vg_grid_desc &g, uint32_t total, bool scratch) {
+static SorPlan sor_block_plan(const vg_grid_desc &g, uint32_t total, bool scratch) {
     const int nx = (int)g.np[0], ny = (int)g.np[1], nz = (int)g.np[2], iy = ny - 2, iz = nz - 2;
     const int chunks = (nx - 2 + kSorChunk - 1) / kSorChunk;
     SorPlan best;
-    auto consider = [&](int by, int bz, int passes, bool whole) {
+    // blocks: how many there are; launches: ceil(total / passes).  (Three
+    // thousand calls: no division that a comparison or a table can spare.)
+    auto consider = [&](int by, int bz, int passes, bool whole, int blocks, double launches) {
         const int halo = whole ? 1 : passes;
         const int ey = std::min(ny, by + 2 * halo), ez = std::min(nz, bz + 2 * halo);
         // kSorChunk floats behind the last row: see the kernel's reads
         const size_t lds = (((size_t)ey * ez + (size_t)(ey - 2) * (ez - 2)) * nx +
                             2 * kSorChunk) * sizeof(float);
         if (lds > kSorLdsBytes) return;
-        SorPlan q;
-        q.by = by;
-        q.bz = bz;
-        q.passes = passes;
-        q.lds = lds;
         const int rows = (ey - 1) / 2 * (ez - 2);
-        q.slot_threads = std::min(kSorThreads, (rows + 63) / 64 * 64);
-        q.slots = std::max(1, std::min(std::min(chunks, passes), kSorThreads / q.slot_threads));
+        const int slot_threads = std::min(kSorThreads, (rows + 63) / 64 * 64);
+        static constexpr int kFit[17] = {0, 16, 8, 5, 4, 3, 2, 2, 2, 1, 1, 1, 1, 1, 1, 1, 1};
+        static_assert(kSorThreads == 1024, "kFit: kSorThreads / 64 waves by waves of a slot");
+        const int slots = std::max(1, std::min(std::min(chunks, passes), kFit[slot_threads / 64]));
+        const int busy = slots * slot_threads;
+        const int groups = 3 * blocks, fit = 2 * lds <= kSorLdsBytes ? 2 : 1;
+        const int share = groups > 256 ? fit : 1;
+        const int rounds = fit == 2 ? (groups + 511) / 512 : (groups + 255) / 256;
+        const int period = std::max(chunks, slots);
+        const int ticks = (passes - 1) / slots * period + (passes - 1) % slots + chunks;
+        const double step = std::max(160.0, 85.0 * share * ((busy / 64 + 3) / 4)) *
+                            (rows <= slot_threads ? 1 : (rows + slot_threads - 1) / slot_threads);
+        const double group_us =
+            lds * 7e-5 * share + ticks * ((400.0 + kSorChunk * step) * (1.0 / 2400.0));
+        const double us = (3.0 + rounds * group_us) * launches + (whole ? 0.0 : 6.0);
+        if (best.by && us >= best.us) return;
+        best.by = by;
+        best.bz = bz;
+        best.passes = passes;
+        best.slots = slots;
+        best.slot_threads = slot_threads;
         // the staging wants every load it can have in flight, the ticks no
         // more waves at their barriers than sweep rows
-        const int busy = q.slots * q.slot_threads;
-        q.threads = whole ? std::max(256, busy) : kSorThreads;
-        const int groups = 3 * ((iy + by - 1) / by) * ((iz + bz - 1) / bz);
-        const int fit = std::min(2, (int)(kSorLdsBytes / lds)), share = groups > 256 ? fit : 1;
-        const int rounds = (groups + 256 * fit - 1) / (256 * fit);
-        const int period = std::max(chunks, q.slots);
-        const int ticks = (passes - 1) / q.slots * period + (passes - 1) % q.slots + chunks;
-        const double step = std::max(160.0, 85.0 * share * ((busy / 64 + 3) / 4)) *
-                            ((rows + q.slot_threads - 1) / q.slot_threads);
-        const double group_us = lds * 7e-5 * share + ticks * (400.0 + kSorChunk * step) / 2400.0;
-        q.us = (3.0 + rounds * group_us) * std::ceil((double)total / passes) + (whole ? 0.0 : 6.0);
-        if (best.by == 0 || q.us < best.us) best = q;
+        best.threads = whole ? std::max(256, busy) : kSorThreads;
+        best.rounds = rounds;
+        best.lds = lds;
+        best.us = us;
     };
-    consider(iy, iz, (int)total, true);
+    consider(iy, iz, (int)total, true, 1, 1.0);
     // one wave per SIMD or fewer: nothing is faster than a single launch
     if (best.by && (size_t)iy * iz <= 512) return best;
-    const int sizes[] = {4, 5, 6, 7, 8, 9, 10, 11, 12, 14, 16, 20, 24, 32};
-    if (scratch)
-        for (int passes : {2, 4, 6, 8})
-            for (int by : sizes)
-                for (int bz : sizes)
-                    if (passes <= (int)total && by <= iy && bz <= iz)
-                        consider(by, bz, passes, false);
+    if (!scratch) return best;
+    static constexpr int kSizes[] = {4, 5, 6, 7, 8, 9, 10, 11, 12, 14, 16, 20, 24, 32};
+    constexpr int kCount = sizeof kSizes / sizeof *kSizes;
+    int ways[2][kCount];
+    for (int i = 0; i < kCount; ++i) {
+        ways[0][i] = (iy + kSizes[i] - 1) / kSizes[i];
+        ways[1][i] = (iz + kSizes[i] - 1) / kSizes[i];
+    }
+    for (int passes : {2, 4, 6, 8}) {
+        if (passes > (int)total) break;
+        const double launches = std::ceil((double)total / passes);
+        for (int i = 0; i < kCount && kSizes[i] <= iy; ++i)
+            for (int j = 0; j < kCount && kSizes[j] <= iz; ++j)
+                consider(kSizes[i], kSizes[j], passes, false, ways[0][i] * ways[1][j], launches);
+    }
     return best;
 }
 
-// The choice takes some tens of microseconds on the host: each thread keeps
-// its last ones (a cascade has about six grids).
-static SorPlan sor_plan_kept(const vg_grid_desc &g, uint32_t total, bool scratch) {
+// A colour pass of the row kernels, in microseconds, fitted to 760 grids of
+// 3x3x3 to 793x77x263 points: launches follow each other every 3.6; a row's
+// chain takes 0.21 a point, up to 0.48 where all of a wave's lanes hold rows,
+// 1.4 times that where waves share a CU, and 0.37 with a lane per component;
+// and all points together 17.5 ns per thousand while the caches hold the
+// fields (129x129x129: 52 us), 24.5 past that (321x321x321: 858), more where
+// the waves' lanes are not full.
+static double sor_rows_us(const vg_grid_desc &g) {
+    const double n = (double)capacity(g), nx = g.np[0];
+    const uint32_t half = (g.np[1] - 1) / 2 + 1;
+    if (nx <= 4) return std::max(3.6, n * 0.011e-3);
+    double slope, mem;
+    if ((size_t)half * (g.np[2] - 2) < kSorSplitRows) {
+        slope = 0.21 + 0.27 * std::max(0, (int)std::min(half, 64u) - 32) / 32.0;
+        if ((size_t)ceil_div(half, 64) * (g.np[2] - 2) > 256) slope *= 1.4;
+        mem = n * 0.020e-3;
+    } else {
+        slope = 0.37;
+        const double full = (double)half / (ceil_div(half, kSorRowsPerWave) * kSorRowsPerWave);
+        const double past = std::min(1.0, std::max(0.0, n - 9e6) / 11e6);
+        mem = n * (0.0175e-3 + 0.007e-3 * past) / std::sqrt(full);
+    }
+    return std::max(std::max(3.6, nx > 6 ? 2.5 + nx * slope : 0.0), mem);
+}
+
+// The grid's plan, or none where the row kernels are faster: few passes, each
+// of a launch's time (33x33x33, one step: 17 us by rows, 20 in blocks), and
+// large grids, whose blocks read many rows around few (321x321x321, 8 steps:
+// 13.7 and 16.2 ms; 129x129x129, 16 steps: 1.66 and 0.96).  Plans of more
+// launches than one also pay for the fields' transposition, 10.7 ns per
+// thousand points, and where the scratch is an allocation of theirs, 23 us of
+// the host's time at least: 250 for one past 2 MiB of another size than the
+// last, which the runtime does not keep (33x41x50 points, one step: 34 us by
+// rows, 146 in blocks), or past 32, which it returns when the stream is waited
+// for; 20 in between.  Rounds of workgroups overlap, so that many take 0.85 of their sum.
+// (On those grids the choice was never below 0.95 of the row kernels' speed
+// nor, with scratch at hand, 0.8 of the blocks', but for a microsecond's host
+// work in solves of one or two launches.)
+static SorPlan sor_plan(const vg_grid_desc &g, uint32_t total, SorScratch scratch) {
+    const double by_rows = sor_rows_us(g) * total;
+    const size_t bytes = 9 * capacity(g) * sizeof(float);
+    double least = 0.0, extra = 0.0;  // the allocation's time, hidden and not
+    if (scratch == SorScratch::Own || scratch == SorScratch::Again) {
+        least = 23.0;
+        if (bytes > size_t(2) << 20)
+            extra = scratch == SorScratch::Own || bytes > size_t(32) << 20 ? 250.0 : 20.0;
+    }
+    const SorPlan q =
+        sor_block_plan(g, total, scratch != SorScratch::None && by_rows > least + extra);
+    if (q.by == 0) return q;
+    double us = q.us * (0.85 + 0.15 / q.rounds);
+    if (!sor_whole(g, q, total)) {
+        if (g.np[0] <= 4) us *= 2.0;  // rows of a few points: the staging's own work
+        us = std::max(us + 0.0107e-3 * (double)capacity(g), least) + extra;
+    }
+    return us * 1.04 < by_rows ? q : SorPlan();
+}
+
+// The choice takes 4 us on the host: each thread keeps its last ones (a
+// cascade has about six grids).
+static SorPlan sor_plan_kept(const vg_grid_desc &g, uint32_t total, SorScratch scratch) {
     struct Kept {
         uint32_t np[3] = {0, 0, 0}, total = 0;
-        bool scratch = false;
+        SorScratch scratch = SorScratch::None;
         SorPlan plan;
     };
     static thread_local Kept kept[16];
@@ -694,13 +778,7 @@ static SorPlan sor_plan_kept(const vg_grid_desc &g, uint32_t total, bool scratch
     return k.plan;
 }
 
-static bool sor_whole(const vg_grid_desc &g, const SorPlan &plan, uint32_t total) {
-    return plan.by > 0 && plan.passes == (int)total && plan.by == (int)g.np[1] - 2 &&
-           plan.bz == (int)g.np[2] - 2;
-}
-
-// The plan of a solve; scratch: whether it may read any.
-static SorPlan sor_plan_of(const vg_grid_desc &g, uint32_t steps, bool scratch) {
+static SorPlan sor_plan_of(const vg_grid_desc &g, uint32_t steps, SorScratch scratch) {
     if (g.np[0] < 3 || g.np[1] < 3 || g.np[2] < 3 || steps == 0) return SorPlan();
     // (an odd row stride and 32-bit offsets: see k_sor_block)
     const bool fits =
@@ -710,7 +788,7 @@ static SorPlan sor_plan_of(const vg_grid_desc &g, uint32_t steps, bool scratch) 
 
 // Floats of scratch that sor_solve reads if it is given them.
 size_t sor_scratch(const vg_grid_desc &g, uint32_t steps) {
-    const SorPlan plan = sor_plan_of(g, steps, true);
+    const SorPlan plan = sor_plan_of(g, steps, SorScratch::Given);
     return plan.by > 0 && !sor_whole(g, plan, 2 * steps) ? 9 * capacity(g) : 0;
 }
 
@@ -734,21 +812,29 @@ vg_status sor_solve(const vg_grid_desc &g, float *soln, const float *lap, uint32
     const SorCoef c = sor_coef(g);
     const size_t n = capacity(g);
     if (scratch_floats < 9 * n) scratch = nullptr;
-    SorPlan plan = sor_plan_of(g, steps, scratch || !capturing(s));
+    static thread_local size_t last = 0;  // grid points of the last solve without
+    SorScratch mode = SorScratch::Given;
+    if (!scratch) {
+        mode = last == n ? SorScratch::Again : SorScratch::Own;
+        last = n;
+    }
+    SorPlan plan = sor_plan_of(g, steps, mode);
     bool whole = sor_whole(g, plan, 2 * steps);
     float *own = nullptr;
     if (plan.by > 0 && !whole && !scratch) {
-        if (salloc((void **)&own, 9 * n * sizeof(float), s) == VG_OK) {
+        if (!capturing(s) && salloc((void **)&own, 9 * n * sizeof(float), s) == VG_OK) {
             scratch = own;
-        } else {  // no memory for it: the solve that needs none
+        } else {  // under capture, or no memory for it: the plan that needs none
             (void)hipGetLastError();
-            plan = sor_plan_of(g, steps, false);
+            plan = sor_plan_of(g, steps, SorScratch::None);
             whole = sor_whole(g, plan, 2 * steps);
         }
     }
     if (plan.by > 0) {
-        VG_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_sor_block),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSorLdsBytes));
+        if (plan.lds > 64 * 1024)  // (what a launch may ask for by itself)
+            VG_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_sor_block),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)kSorLdsBytes));
         SorBlock b;
         b.nx = (int)g.np[0];
         b.ny = (int)g.np[1];
@@ -763,10 +849,12 @@ vg_status sor_solve(const vg_grid_desc &g, float *soln, const float *lap, uint32
         if (whole) {
             b.in_mul = b.out_mul = b.f_mul = 3;
             b.in_comp = b.out_comp = b.f_comp = 1;
-            // about a millisecond a launch at most
-            constexpr uint32_t kMost = 1024;
-            for (uint32_t done = 0; done < 2 * steps && st == VG_OK; done += kMost) {
-                b.passes = (int)std::min(kMost, 2 * steps - done);
+            // about a millisecond a launch at most, by the plan's estimate (1025x5x5:
+            // 10 us a pass), of an even number of passes: each starts with colour 0
+            const double most = 500.0 * 2 * steps / plan.us;
+            const uint32_t per = 2 * (uint32_t)std::max(1.0, std::min(most, 1e6));
+            for (uint32_t done = 0; done < 2 * steps && st == VG_OK; done += per) {
+                b.passes = (int)std::min(per, 2 * steps - done);
                 b.color = 0;
                 st = launch("vg_sor_block", k_sor_block, grid, block, plan.lds, s, b,
                             (const float *)soln, soln, lap, c);
