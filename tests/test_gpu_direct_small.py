@@ -32,3 +32,31 @@ def test_fine_blocks(vg, oracle, n, nq, policy):
         want = cpu(pos, om, size, pts, 1.3, 0.7, policy=policy, threads=8)
         # FP32 terms of random sign summed in another order
         assert np.linalg.norm(out.numpy() - want) <= 1e-5 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("partials", [1, 15, 16, 17, 32, 33, 2000])
+def test_partials_of_many_tiles(vg, oracle, partials):
+    """A tile per workgroup and their sum, which takes 16 of them at a time:
+    the edges of those, and the time of many (few queries by many vortons)."""
+    n, nq = 256 * partials, 64
+    print(f"[case] direct sum, {partials} partials", flush=True)
+    rng = np.random.default_rng(partials)
+    pos, om, q = (rng.normal(size=(k, 3)).astype(F32) for k in (n, n, nq))
+    dp, dw, dq = (vg.DeviceArray.from_numpy(a) for a in (pos, om, q))
+    v = vg.vortons_view(dp, dw, n, uniform_size=0.2)
+    out = vg.DeviceArray.zeros((nq, 3))
+    vg.direct_velocity(v, dq, nq, out, policy=1)
+    vg.profile_reset()
+    vg.profile_enable(True)
+    try:
+        vg.direct_velocity(v, dq, nq, out, policy=1)
+        vg.synchronize()
+        ms, _ = vg.profile_get("vg_direct_reduce")
+    finally:
+        vg.profile_enable(False)
+    want = oracle.direct_velocity_f64(pos, om, np.full(n, 0.2, F32), q, threads=8)
+    # FP32 terms of random sign; 64-bit sums, which a serial FP32 one of
+    # 512,000 terms misses by 1.3e-5
+    assert np.linalg.norm(out.numpy() - want) <= 1e-5 * np.linalg.norm(want)
+    # 2000 partials: 75 us with 16 loads under way, 480 with one
+    assert ms < 0.2
