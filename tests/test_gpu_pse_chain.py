@@ -52,3 +52,53 @@ def test_slices_past_the_lds(vg, oracle):
     og = oracle.define_shape(int(np.prod(cells)), np.zeros(3), ext, pow2=False)
     assert og.shape == tuple(c + 1 for c in cells)
     run(vg, oracle, og, pos, om, 0.02, rng)
+
+
+def kernels(vg, f):
+    vg.profile_reset()
+    vg.profile_enable(True)
+    try:
+        f()
+        return {k for k in vg.profile_dump() if k.startswith("vg_pse_")}
+    finally:
+        vg.profile_enable(False)
+
+
+@pytest.mark.parametrize("cells", [(513, 257, 1), (514, 258, 2), (512, 256, 1)])
+@pytest.mark.parametrize("fractions", [None, "0"])
+def test_flat_grids(vg, oracle, monkeypatch, cells, fractions):
+    """Wavefront steps of more cells than the schedule deals, and of as many:
+    cells of no vortons up to two chunks, with the fractions precomputed and in
+    the serial exchange."""
+    print(f"[case] PSE flat grid {cells}, fractions {fractions}", flush=True)
+    if fractions is not None:
+        monkeypatch.setenv("VG_PSE_FRACTIONS", fractions)
+    rng = np.random.default_rng(sum(cells))
+    h = 0.05
+    ext = np.array(cells) * h
+    pos = [rng.uniform(0.0005, 0.9995, (40000, 3)) * ext]
+    for k in (3, 4, 5, 63, 64, 65, 130):
+        at = np.array([rng.integers(c) for c in cells])
+        pos.append((at + rng.uniform(0.1, 0.9, (k, 3))) * h)
+    pos = np.concatenate(pos).astype(F32)
+    om = rng.normal(size=pos.shape).astype(F32)
+    og = oracle.define_shape(int(np.prod(cells)), np.zeros(3), ext, pow2=False)
+    assert og.shape == tuple(c + 1 for c in cells)
+    ran = kernels(vg, lambda: run(vg, oracle, og, pos, om, 0.04, rng))
+    assert ("vg_pse_fractions" in ran) == (fractions is None)
+    assert ("vg_pse_schedule" in ran) == (cells == (512, 256, 1))
+
+
+@pytest.mark.parametrize("blob", [2401, 5000])
+def test_cells_past_the_chain_keep_precomputed_fractions(vg, oracle, blob):
+    """Cells of one wave's share of the fractions beside one of many."""
+    print(f"[case] PSE fractions by rows, a cell of {blob} vortons", flush=True)
+    rng = np.random.default_rng(blob)
+    cells, h = (9, 8, 7), 0.25
+    ext = np.array(cells) * h
+    lump = (np.array([4, 3, 2]) + rng.uniform(0.1, 0.9, (blob, 3))) * h
+    pos = np.concatenate([rng.uniform(0.002, 0.998, (9000, 3)) * ext, lump]).astype(F32)
+    om = rng.normal(size=pos.shape).astype(F32)
+    og = oracle.define_shape(int(np.prod(cells)), np.zeros(3), ext, pow2=False)
+    assert og.shape == tuple(c + 1 for c in cells)
+    assert "vg_pse_fractions" in kernels(vg, lambda: run(vg, oracle, og, pos, om, 0.2, rng))

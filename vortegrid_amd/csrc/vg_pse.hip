@@ -28,7 +28,7 @@
 // A cell's exchanges are a serial chain, and the chains are what the call
 // waits for: 47k systolic steps (pse_cell_chain) in 540 cells on the slowest
 // slices of the two phases at 1M vortons (129^3), 16.5 ms when a step moved
-// all of Omega and its index down the lanes and stored through memory, 3.8
+// all of Omega and its index down the lanes and stored through memory, 3.4
 // ms now.  So a step carries as little as it can:
 //   * the exchange fraction f of a pair depends on positions and sizes only:
 //     k_pse_fractions computes all of them over the whole chip beforehand, in
@@ -41,9 +41,16 @@
 // The vorton state lives in the tree's cell-sorted order (positions and
 // sizes from the tree, angular velocities gathered from the caller and
 // scattered back), so a cell's vortons are contiguous.  exp is vg_pse_exp,
-// the same function as the oracle's.  Cells with more than kChainPartners
-// partners, or fractions that would fill 8 GB, take the form with the
-// fractions in the chain (k_pse_phase).
+// the same function as the oracle's.
+//
+// The form is chosen for the whole call: one cell of more than kChainPartners
+// partners, a wavefront step of more cells than k_pse_schedule deals (flat
+// grids from 513x257 cells) or 8 GB of fractions or more give it k_pse_phase,
+// whose steps move all of Omega, with the fractions precomputed by rows
+// (k_pse_row_fractions) or, where those fill 8 GB too, formed in the chain:
+// 1M vortons with 8 cells of 320 take 20.3 ms (24.7 when one wave formed each
+// cell's fractions, 28.2 with them in the chain), 8M in 700x300x8 cells 749
+// (1148 in the chain).
 #include <cstdlib>
 
 #include "vg_internal.h"
@@ -113,6 +120,11 @@ struct PseArgs {
     const float4 *p;                // sorted (x, y, z, size)
     float4 *w;                      // sorted (Omega, alive)
     float nu_dt2, dissipation;
+    // k_pse_phase's exchange fractions of the systolic cells, precomputed (or
+    // null): the cell with leaf point c holds frac[frac_off[c] + i n + j] for
+    // here-vorton i < k and partner j < n (0 where j <= i).
+    const float *frac;
+    const uint32_t *frac_off;
 };
 
 __device__ __forceinline__ void pse_cell(const PseArgs &a, uint32_t x, uint32_t y, uint32_t z) {
@@ -249,6 +261,101 @@ __device__ __forceinline__ void pse_cell_systolic(const PseArgs &a, const uint32
     }
 }
 
+// Lane l takes lane l + 1 (wrapping): the whole-wave DPP rotation
+// (wave_rol:1), so the window's next partner is always in lane 0.
+__device__ __forceinline__ float wave_rol(float v) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x134, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float4 wave_rol4(float4 v) {
+    return make_float4(wave_rol(v.x), wave_rol(v.y), wave_rol(v.z), wave_rol(v.w));
+}
+__device__ __forceinline__ uint32_t wave_rol_u(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x134, 0xf, 0xf, false);
+}
+__device__ __forceinline__ uint32_t wave_shr_u(uint32_t v, uint32_t in) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)in, (int)v, 0x138, 0xf, 0xf, false);
+}
+
+// The systolic cell with its fractions read from a.frac: only Omega (and
+// its vorton's index, for the write-back of partners leaving the last lane)
+// streams down the lanes.  The window of 64 loaded partners rotates by one
+// lane per step, so lane 0 always holds the next partner to enter; each
+// lane's fractions are loaded kFracAhead steps before use (a lane walks its
+// row of the fraction block left to right).
+constexpr int kFracAhead = 8;
+
+__device__ __forceinline__ void pse_cell_systolic_frac(const PseArgs &a, uint32_t c,
+                                                       const uint32_t base[8],
+                                                       const uint32_t pre[9], uint32_t k,
+                                                       uint32_t n) {
+#pragma clang fp contract(off)
+    const int lane = (int)(threadIdx.x & 63);
+    const float *__restrict__ fc = a.frac + a.frac_off[c];
+    for (uint32_t B = 0; B < k; B += 64) {
+        const uint32_t L = k - B < 64u ? k - B : 64u;
+        const uint32_t i = B + (uint32_t)lane;
+        const uint32_t gi = base[0] + i;  // here-vortons are the cell's own
+        float4 wh = make_float4(0.f, 0.f, 0.f, 0.f), sw = wh, bw = wh;
+        uint32_t sg = 0, bg = 0;
+        bool live = false;
+        const uint32_t steps = (n - B) + L - 1;
+        // fraction of this lane at step t (0 unless it exchanges then)
+        auto fetch = [&](uint32_t t) -> float {
+            const int jl = (int)t - lane;
+            const uint32_t j = B + (uint32_t)jl;
+            return ((uint32_t)lane < L && jl > lane && j < n) ? fc[(size_t)i * n + j] : 0.f;
+        };
+        float cur[kFracAhead], nxt[kFracAhead];
+#pragma unroll
+        for (int d = 0; d < kFracAhead; ++d) cur[d] = fetch((uint32_t)d);
+        for (uint32_t t0 = 0; t0 < steps; t0 += kFracAhead) {
+#pragma unroll
+            for (int d = 0; d < kFracAhead; ++d) nxt[d] = fetch(t0 + kFracAhead + (uint32_t)d);
+#pragma unroll
+            for (int d = 0; d < kFracAhead; ++d) {
+                const uint32_t t = t0 + (uint32_t)d;
+                if (t >= steps) break;
+                if ((t & 63u) == 0) {  // the next 64 partners to enter, one per lane
+                    const uint32_t jj = B + t + (uint32_t)lane;
+                    if (jj < n) {
+                        bg = partner_index(base, pre, jj);
+                        bw = a.w[bg];
+                    }
+                }
+                sw = wave_shr4(sw, bw);  // lane 0 takes the window's lane 0
+                sg = wave_shr_u(sg, bg);
+                bw = wave_rol4(bw);
+                bg = wave_rol_u(bg);
+                const int jl = (int)t - lane;  // partner j - B at this lane
+                const uint32_t j = B + (uint32_t)jl;
+                if ((uint32_t)lane < L && jl >= 0 && j < n) {
+                    if (jl == lane) {  // j == i: the here-vorton itself
+                        wh = sw;
+                        live = sw.w != 0.f;
+                    } else if (jl > lane && live) {
+                        exchange_f(wh, sw, cur[d]);
+                    }
+                    if (j == n - 1) {  // the lane's last partner: done
+                        if (live) {
+                            wh.x -= wh.x * a.dissipation;
+                            wh.y -= wh.y * a.dissipation;
+                            wh.z -= wh.z * a.dissipation;
+                        }
+                        a.w[gi] = wh;
+                    }
+                    // a partner that is not a here-vorton of this chunk leaves
+                    // the last lane with its value for the next chunk
+                    if ((uint32_t)lane == L - 1 && j >= B + L) a.w[sg] = sw;
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < kFracAhead; ++d) cur[d] = nxt[d];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    }
+}
+
 __device__ __forceinline__ void pse_cell_wave(const PseArgs &a, uint32_t x, uint32_t y, uint32_t z) {
 #pragma clang fp contract(off)
     const int lane = (int)(threadIdx.x & 63);
@@ -265,7 +372,10 @@ __device__ __forceinline__ void pse_cell_wave(const PseArgs &a, uint32_t x, uint
     const uint32_t k = pre[1], n = pre[8];
     if (k == 0) return;
     if (k >= kSystolicMin) {
-        pse_cell_systolic(a, base, pre, k, n);
+        if (a.frac)
+            pse_cell_systolic_frac(a, c, base, pre, k, n);
+        else
+            pse_cell_systolic(a, base, pre, k, n);
         return;
     }
     if (n > 64u * kSlots) {
@@ -380,16 +490,23 @@ __device__ __forceinline__ uint32_t chunk_groups(uint32_t n, uint32_t B, uint32_
     return ((n - B) + L - 1 + 3) / 4;
 }
 
-// Fractions (floats) of each leaf point's cell, their 64-bit sum, the largest
-// partner count and the largest number of vortons in two adjacent slices
-// (totals[0..2]).  A grid-stride loop: with one workgroup per 256 points the
+// Floats of a cell's fractions by rows (PseArgs::frac): those of the systolic
+// cells only.
+__device__ __forceinline__ unsigned long long row_fractions(uint32_t k, uint32_t n) {
+    return k >= kSystolicMin ? (unsigned long long)k * n : 0ull;
+}
+
+// Fractions (floats) of each leaf point's cell in the chain's order, their
+// 64-bit sum, the largest partner count, the largest number of vortons in two
+// adjacent slices, and the sum by rows (totals[0..3]).  A grid-stride loop: with one workgroup per 256 points the
 // two atomics of each took 157 us at 129^3.
 __global__ __launch_bounds__(256) void k_pse_frac_size(PseArgs a, uint32_t cells, uint32_t n_all,
                                                        uint32_t *__restrict__ size,
                                                        unsigned long long *__restrict__ totals) {
     __shared__ unsigned long long part[256];
+    __shared__ unsigned long long part_rows[256];
     __shared__ uint32_t most[256];
-    unsigned long long sum = 0;
+    unsigned long long sum = 0, rows = 0;
     uint32_t widest = 0;
     for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < cells;
          c += gridDim.x * blockDim.x) {
@@ -402,22 +519,26 @@ __global__ __launch_bounds__(256) void k_pse_frac_size(PseArgs a, uint32_t cells
                 f += 4ull * L * chunk_groups(n, B, L);
             }
             widest = max(widest, n);
+            rows += row_fractions(k, n);
         }
         size[c] = f < 0x80000000ull ? (uint32_t)f : 0x80000000u;
         sum += f;
     }
     part[threadIdx.x] = sum;
+    part_rows[threadIdx.x] = rows;
     most[threadIdx.x] = widest;
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
         if ((int)threadIdx.x < w) {
             part[threadIdx.x] += part[threadIdx.x + w];
+            part_rows[threadIdx.x] += part_rows[threadIdx.x + w];
             most[threadIdx.x] = max(most[threadIdx.x], most[threadIdx.x + w]);
         }
         __syncthreads();
     }
     if (threadIdx.x == 0 && part[0]) {
         atomicAdd(&totals[0], part[0]);
+        atomicAdd(&totals[3], part_rows[0]);
         atomicMax(&totals[1], (unsigned long long)most[0]);
     }
     if (blockIdx.x == 0) {
@@ -425,6 +546,65 @@ __global__ __launch_bounds__(256) void k_pse_frac_size(PseArgs a, uint32_t cells
         for (uint32_t z = threadIdx.x; z + 1 < a.nz; z += blockDim.x)
             pair = max(pair, slice_pair(a, z, n_all).count);
         atomicMax(&totals[2], (unsigned long long)pair);
+    }
+}
+
+// The fractions' sizes by rows, and which cells have more than one wave
+// computes (wide[0] of them from wide[1] on, in no order).
+constexpr uint32_t kRowsPerWave = 1u << 16;
+__global__ __launch_bounds__(256) void k_pse_row_size(PseArgs a, uint32_t cells,
+                                                      uint32_t *__restrict__ size,
+                                                      uint32_t *__restrict__ wide) {
+    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= cells) return;
+    const uint32_t k = a.count[c];
+    const uint32_t f =
+        k >= kSystolicMin ? (uint32_t)row_fractions(k, cell_partners(a, c).pre[8]) : 0u;
+    size[c] = f;
+    if (f > kRowsPerWave) wide[1 + atomicAdd(&wide[0], 1u)] = c;
+}
+
+// A cell's fractions by rows, every `stride`th from `first` on: the same
+// operations as the in-chain exchange, so the same bits.
+__device__ __forceinline__ void row_fractions_of(const PseArgs &a, uint32_t c,
+                                                 const CellPartners &cp, uint32_t first,
+                                                 uint32_t stride, float *__restrict__ frac) {
+#pragma clang fp contract(off)
+    const uint32_t n = cp.pre[8], total = cp.pre[1] * n;  // (below 2^31: the sum of them is)
+    float *__restrict__ fc = frac + a.frac_off[c];
+    for (uint32_t q = first; q < total; q += stride) {
+        const uint32_t i = q / n, j = q - i * n;
+        float f = 0.f;
+        if (j > i) {
+            const float4 ph = a.p[cp.base[0] + i];
+            const float range = 4.0f * ph.w;
+            f = pse_fraction(ph, range * range, a.p[partner_index(cp.base, cp.pre, j)], a.nu_dt2);
+        }
+        fc[q] = f;
+    }
+}
+
+// One wave per leaf point's cell, and kWideParts workgroups for the cells past
+// that: with one wave for those, too, a cell of 6,000 vortons took 222 ms a
+// call instead of 103.
+constexpr uint32_t kWideParts = 64;
+__global__ __launch_bounds__(256) void k_pse_row_fractions(PseArgs a, uint32_t cells,
+                                                           float *__restrict__ frac) {
+    const uint32_t c = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (c >= cells) return;
+    const uint32_t k = a.count[c];
+    if (k < kSystolicMin) return;
+    const CellPartners cp = cell_partners(a, c);
+    if (row_fractions(k, cp.pre[8]) <= kRowsPerWave)
+        row_fractions_of(a, c, cp, threadIdx.x & 63, 64, frac);
+}
+__global__ __launch_bounds__(256) void k_pse_row_fractions_wide(PseArgs a,
+                                                                const uint32_t *__restrict__ wide,
+                                                                float *__restrict__ frac) {
+    for (uint32_t w = blockIdx.x / kWideParts; w < wide[0]; w += gridDim.x / kWideParts) {
+        const uint32_t c = wide[1 + w];
+        row_fractions_of(a, c, cell_partners(a, c), blockIdx.x % kWideParts * 256 + threadIdx.x,
+                         kWideParts * 256, frac);
     }
 }
 
@@ -1053,6 +1233,8 @@ vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const 
     a.w = w;
     a.nu_dt2 = 2.0f * viscosity * dt;   // 2.0f * mViscosity * timeStep
     a.dissipation = viscosity * dt;     // mViscosity * timeStep
+    a.frac = nullptr;
+    a.frac_off = nullptr;
     if (sim) {
         vg_status st = launch("vg_pse_gather", k_pse_gather, dim3(ceil_div(n, 256)), dim3(256), 0,
                               s, tv.sorted_idx, (const float *)angvel, ang_stride, birth,
@@ -1073,7 +1255,7 @@ vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const 
     const uint32_t M = cy < (cx + 1) / 2 ? cy : (cx + 1) / 2;
     const size_t nsched = (size_t)slices * steps, cells = capacity(g);
     uint32_t *perm = nullptr, *wstart = nullptr, *fsize = nullptr, *foff = nullptr,
-             *stmp = nullptr, *list = nullptr, *lstart = nullptr;
+             *stmp = nullptr, *list = nullptr, *lstart = nullptr, *wide = nullptr;
     unsigned long long *dtot = nullptr;
     float *frac = nullptr;
     // The fractions' sizes are read back to size their buffer: one stream
@@ -1081,14 +1263,14 @@ vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const 
     vg_status st = salloc((void **)&fsize, cells * sizeof(uint32_t), s);
     if (st == VG_OK) st = salloc((void **)&foff, cells * sizeof(uint32_t), s);
     if (st == VG_OK) st = salloc((void **)&stmp, scan_scratch_elems(cells) * sizeof(uint32_t), s);
-    if (st == VG_OK) st = salloc((void **)&dtot, 3 * sizeof(unsigned long long), s);
-    if (st == VG_OK) st = launch("vg_pse_frac_size", k_pse_zero64, dim3(1), dim3(3), 0, s, dtot);
+    if (st == VG_OK) st = salloc((void **)&dtot, 4 * sizeof(unsigned long long), s);
+    if (st == VG_OK) st = launch("vg_pse_frac_size", k_pse_zero64, dim3(1), dim3(4), 0, s, dtot);
     if (st == VG_OK)
         st = launch("vg_pse_frac_size", k_pse_frac_size,
                     dim3(min(ceil_div(cells, 256), 1024u)), dim3(256), 0, s, a, (uint32_t)cells,
                     (uint32_t)n, fsize, dtot);
     if (st == VG_OK) st = exclusive_scan_u32(fsize, foff, cells, stmp, s);
-    unsigned long long totals[3] = {0, 0, 0};
+    unsigned long long totals[4] = {0, 0, 0, 0};
     if (st == VG_OK) {
         hipError_t e = hipMemcpyAsync(totals, dtot, sizeof totals, hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -1097,13 +1279,16 @@ vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const 
             st = VG_EDEVICE;
         }
     }
-    // Fractions of 2^31 floats or more, and cells whose partners do not fit
-    // a wave's LDS, keep the fractions in the chain, and so does
-    // VG_PSE_FRACTIONS=0 in the environment (the same bits either way; the
-    // switch keeps that path testable).
+    // One cell whose partners do not fit a wave's LDS, a wavefront step of more
+    // cells than the schedule deals, or 2^31 floats of fractions or more keep
+    // the whole call in the form without the chain; it reads its fractions by
+    // rows, unless those are 2^31 floats or more, too.  VG_PSE_FRACTIONS=0 in
+    // the environment keeps them in the serial exchange (the same bits any
+    // way; the switch keeps that path testable).
     const char *env = getenv("VG_PSE_FRACTIONS");
+    const bool precompute = !(env && env[0] == '0');
     const bool scheduled = M <= 64u * kSchedSlots && nsched * M < (size_t(1) << 28);
-    const bool chain = !(env && env[0] == '0') && totals[0] > 0 && totals[0] < (1ull << 31) &&
+    const bool chain = precompute && totals[0] > 0 && totals[0] < (1ull << 31) &&
                        totals[1] <= kChainPartners && scheduled && steps < (1u << 16);
     const uint32_t waves = chain ? kChainWaves : kPseWaves;
     if (st == VG_OK && scheduled) {
@@ -1158,6 +1343,25 @@ vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const 
             st = launch("vg_pse_gather", k_pse_gather, dim3(ceil_div(n, 256)), dim3(256), 0, s,
                         tv.sorted_idx, (const float *)angvel, ang_stride, birth, birth_stride, n,
                         w);
+        if (st == VG_OK && precompute && totals[3] > 0 && totals[3] < (1ull << 31)) {
+            // (the cells past one wave's share: fewer than the fractions hold of it)
+            const size_t most = 1 + totals[3] / kRowsPerWave;
+            st = salloc((void **)&wide, (1 + most) * sizeof(uint32_t), s);
+            if (st == VG_OK) st = zero_fill(wide, sizeof(uint32_t), s);
+            if (st == VG_OK)
+                st = launch("vg_pse_frac_size", k_pse_row_size, dim3(ceil_div(cells, 256)),
+                            dim3(256), 0, s, a, (uint32_t)cells, fsize, wide);
+            if (st == VG_OK) st = exclusive_scan_u32(fsize, foff, cells, stmp, s);
+            if (st == VG_OK) st = salloc((void **)&frac, totals[3] * sizeof(float), s);
+            a.frac = frac;
+            a.frac_off = foff;
+            if (st == VG_OK)
+                st = launch("vg_pse_fractions", k_pse_row_fractions, dim3(ceil_div(cells, 4)),
+                            dim3(256), 0, s, a, (uint32_t)cells, frac);
+            if (st == VG_OK && totals[1] * totals[1] > kRowsPerWave)
+                st = launch("vg_pse_fractions", k_pse_row_fractions_wide, dim3(32 * kWideParts),
+                            dim3(256), 0, s, a, (const uint32_t *)wide, frac);
+        }
         for (uint32_t phase = 0; phase < 2 && st == VG_OK; ++phase) {
             const uint32_t groups = (slices - phase + 1) / 2;
             if (groups)
@@ -1172,6 +1376,7 @@ vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const 
     if (wstart) sfree(wstart, s);
     if (list) sfree(list, s);
     if (lstart) sfree(lstart, s);
+    if (wide) sfree(wide, s);
     if (frac) sfree(frac, s);
     if (fsize) sfree(fsize, s);
     if (foff) sfree(foff, s);
