@@ -102,3 +102,33 @@ def test_cells_past_the_chain_keep_precomputed_fractions(vg, oracle, blob):
     og = oracle.define_shape(int(np.prod(cells)), np.zeros(3), ext, pow2=False)
     assert og.shape == tuple(c + 1 for c in cells)
     assert "vg_pse_fractions" in kernels(vg, lambda: run(vg, oracle, og, pos, om, 0.2, rng))
+
+
+@pytest.mark.parametrize("dead", [0.4, 0.95])
+def test_zeros_keep_their_sign(vg, oracle, dead):
+    """Components of -0 and +0 beside others, in cells of one vorton up to two
+    chunks: alone, adopted, exchanged, and past dead vortons; the bits of the
+    oracle's, not their values."""
+    print(f"[case] PSE signed zeros, {dead} dead", flush=True)
+    rng = np.random.default_rng(5)
+    cells, h = (10, 8, 6), 0.25
+    ext = np.array(cells) * h
+    lumps = [(np.array([rng.integers(c) for c in cells]) + rng.uniform(0.1, 0.9, (k, 3))) * h
+             for k in (1, 2, 3, 64, 70)]
+    pos = np.concatenate([rng.uniform(0.002, 0.998, (400, 3)) * ext] + lumps).astype(F32)
+    om = rng.normal(size=pos.shape).astype(F32)
+    om[rng.random(om.shape) < 0.4] = F32(-0.0)
+    om[rng.random(om.shape) < 0.1] = F32(0.0)
+    og = oracle.define_shape(int(np.prod(cells)), np.zeros(3), ext, pow2=False)
+    assert og.shape == tuple(c + 1 for c in cells)
+    birth = np.where(rng.random(len(pos)) < dead, -1, 5).astype(np.int32)
+    want = oracle.pse_diffuse(og, pos, om, 0.02, 0.5, 0.2, alive=birth >= 0)
+    # (what a live vorton touches loses it: dead ones have it)
+    assert np.count_nonzero((want == 0) & np.signbit(want)) > 10
+    dp, dw = vg.DeviceArray.from_numpy(pos), vg.DeviceArray.from_numpy(om)
+    db = vg.DeviceArray.from_numpy(birth)
+    t = vg.Tree()
+    t.build(vg.GridDesc.from_fields(og), vg.vortons_view(dp, dw, len(pos), uniform_size=0.02))
+    t.pse_diffuse(dw, 0.5, 0.2, birth=db, birth_stride=1)
+    vg.synchronize()
+    assert np.array_equal(dw.numpy().view(np.uint32), want.view(np.uint32))

@@ -52,6 +52,7 @@
 // cell's fractions, 28.2 with them in the chain), 8M in 700x300x8 cells 749
 // (1148 in the chain).
 #include <cstdlib>
+#include <type_traits>
 
 #include "vg_internal.h"
 
@@ -610,7 +611,7 @@ __global__ __launch_bounds__(256) void k_pse_row_fractions_wide(PseArgs a,
 
 // What a lane does at a step of the chain: exchange with the fraction (|f|
 // <= 0.5, or NaN), adopt the incoming value as its here-vorton (kAdopt: an
-// exchange at f = 1 from Omega_h = 0 gives Omega_h = Omega_t exactly), or
+// exchange at f = 1 from Omega_h = -0 gives Omega_h = Omega_t exactly), or
 // nothing (kSkip).
 constexpr float kAdopt = 1.0f, kSkip = -1.0f;
 
@@ -738,39 +739,55 @@ __device__ __forceinline__ void pse_cell_chain(const PseArgs &a, const ChainCell
         // lanes past the last follow it (they receive what leaves it)
         const uint32_t ll = lane < L ? lane : L - 1;
         const bool leaves = lane == L - 1;
-        float wh = 0.f, sw = 0.f;
+        float wh = -0.f, sw = 0.f;
         float4 in = *reinterpret_cast<const float4 *>(buf + B);
         float *out = buf + B - (L - 1);  // of the value leaving at step 0
-        uint32_t g0 = 0;
-        do {
+        // DEAD: the chunk has dead here-vortons, and what passes them keeps its
+        // bits, the sign of a zero among them.  Where all are alive a skipped
+        // value is read no more, and one select instead of two does (3.97
+        // against 3.88 ms a vorticity update at 1M vortons).
+        auto steps = [&](auto DEAD) {
+            uint32_t g0 = 0;
+            do {
 #pragma unroll
-            for (uint32_t r = 0; r < kRing; ++r) {
-                const uint32_t g = g0 + r;
-                if (g < groups) {
-                    const float f[4] = {q[r].x, q[r].y, q[r].z, q[r].w};
-                    const float v[4] = {in.x, in.y, in.z, in.w};
-                    in = *reinterpret_cast<const float4 *>(buf + B + 4 * (g + 1));
-                    float o[4];
+                for (uint32_t r = 0; r < kRing; ++r) {
+                    const uint32_t g = g0 + r;
+                    if (g < groups) {
+                        const float f[4] = {q[r].x, q[r].y, q[r].z, q[r].w};
+                        const float v[4] = {in.x, in.y, in.z, in.w};
+                        in = *reinterpret_cast<const float4 *>(buf + B + 4 * (g + 1));
+                        float o[4];
 #pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        sw = wave_shr(sw, v[d]);  // lane 0 takes the next partner
-                        const float e = (wh - sw) * f[d];
-                        const float ex = f[d] != kSkip ? e : 0.f;
-                        wh -= ex;
-                        sw += ex;
-                        o[d] = sw;
+                        for (int d = 0; d < 4; ++d) {
+                            sw = wave_shr(sw, v[d]);  // lane 0 takes the next partner
+                            const float e = (wh - sw) * f[d];
+                            const bool go = f[d] != kSkip;
+                            if (DEAD) {
+                                wh = go ? wh - e : wh;
+                                sw = go ? sw + e : sw;
+                            } else {
+                                const float ex = go ? e : 0.f;
+                                wh -= ex;
+                                sw += ex;
+                            }
+                            o[d] = sw;
+                        }
+                        // values below B belong to steps before the first partner
+                        // has passed; their places in buf are no longer read
+                        if (4 * g + 3 >= L - 1 && leaves) {
+#pragma unroll
+                            for (int d = 0; d < 4; ++d) out[4 * g + d] = o[d];
+                        }
                     }
-                    // values below B belong to steps before the first partner
-                    // has passed; their places in buf are no longer read
-                    if (4 * g + 3 >= L - 1 && leaves) {
-#pragma unroll
-                        for (int d = 0; d < 4; ++d) out[4 * g + d] = o[d];
-                    }
+                    q[r] = F[min(g + kRing, groups - 1) * L + ll];
                 }
-                q[r] = F[min(g + kRing, groups - 1) * L + ll];
-            }
-            g0 += kRing;
-        } while (g0 < groups);
+                g0 += kRing;
+            } while (g0 < groups);
+        };
+        if (__ballot(lead.live == 0.f))
+            steps(std::true_type());
+        else
+            steps(std::false_type());
         F += groups * L;
         if (lead.live != 0.f) wh -= wh * a.dissipation;
         if (lane < L) w[cp.base[0] + B + lane] = wh;
