@@ -1271,23 +1271,29 @@ vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const 
     // cells per wavefront step are at most min(cy, (cx + 1) / 2)
     const uint32_t M = cy < (cx + 1) / 2 ? cy : (cx + 1) / 2;
     const size_t nsched = (size_t)slices * steps, cells = capacity(g);
-    uint32_t *perm = nullptr, *wstart = nullptr, *fsize = nullptr, *foff = nullptr,
-             *stmp = nullptr, *list = nullptr, *lstart = nullptr, *wide = nullptr;
-    unsigned long long *dtot = nullptr;
+    // (An allocation and its release are 8 us of the host's: what is needed at
+    // one time is one.  100 vortons in 16x16x16 cells: 227 us a call with ten
+    // allocations, 105 with four.)
+    uint32_t *sizes = nullptr, *sched = nullptr, *wide = nullptr;
     float *frac = nullptr;
     // The fractions' sizes are read back to size their buffer: one stream
     // synchronisation.
-    vg_status st = salloc((void **)&fsize, cells * sizeof(uint32_t), s);
-    if (st == VG_OK) st = salloc((void **)&foff, cells * sizeof(uint32_t), s);
-    if (st == VG_OK) st = salloc((void **)&stmp, scan_scratch_elems(cells) * sizeof(uint32_t), s);
-    if (st == VG_OK) st = salloc((void **)&dtot, 4 * sizeof(unsigned long long), s);
-    if (st == VG_OK) st = launch("vg_pse_frac_size", k_pse_zero64, dim3(1), dim3(4), 0, s, dtot);
+    constexpr size_t kTotals = 4;
+    vg_status st = salloc((void **)&sizes,
+                          kTotals * sizeof(unsigned long long) +
+                              (2 * cells + scan_scratch_elems(cells)) * sizeof(uint32_t),
+                          s);
+    unsigned long long *dtot = reinterpret_cast<unsigned long long *>(sizes);
+    uint32_t *fsize = reinterpret_cast<uint32_t *>(dtot + kTotals), *foff = fsize + cells,
+             *stmp = foff + cells;
+    if (st == VG_OK) st = launch("vg_pse_frac_size", k_pse_zero64, dim3(1), dim3(kTotals), 0, s,
+                                  dtot);
     if (st == VG_OK)
         st = launch("vg_pse_frac_size", k_pse_frac_size,
                     dim3(min(ceil_div(cells, 256), 1024u)), dim3(256), 0, s, a, (uint32_t)cells,
                     (uint32_t)n, fsize, dtot);
     if (st == VG_OK) st = exclusive_scan_u32(fsize, foff, cells, stmp, s);
-    unsigned long long totals[4] = {0, 0, 0, 0};
+    unsigned long long totals[kTotals] = {0, 0, 0, 0};
     if (st == VG_OK) {
         hipError_t e = hipMemcpyAsync(totals, dtot, sizeof totals, hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -1308,9 +1314,15 @@ vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const 
     const bool chain = precompute && totals[0] > 0 && totals[0] < (1ull << 31) &&
                        totals[1] <= kChainPartners && scheduled && steps < (1u << 16);
     const uint32_t waves = chain ? kChainWaves : kPseWaves;
+    uint32_t *perm = nullptr, *wstart = nullptr, *list = nullptr, *lstart = nullptr;
     if (st == VG_OK && scheduled) {
-        st = salloc((void **)&perm, nsched * M * sizeof(uint32_t), s);
-        if (st == VG_OK) st = salloc((void **)&wstart, nsched * (waves + 1) * sizeof(uint32_t), s);
+        const size_t deal = nsched * M, starts = nsched * (waves + 1);
+        const size_t lists = chain ? deal + slices * (kChainWaves + 1) : 0;
+        st = salloc((void **)&sched, (deal + starts + lists) * sizeof(uint32_t), s);
+        perm = sched;
+        wstart = perm + deal;
+        list = wstart + starts;
+        lstart = list + deal;
         if (st == VG_OK)
             st = launch("vg_pse_schedule",
                         chain ? k_pse_schedule<kChainWaves, true> : k_pse_schedule<kPseWaves, false>,
@@ -1318,9 +1330,6 @@ vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const 
     }
     if (chain) {
         float *w3 = reinterpret_cast<float *>(w), *alive = w3 + 3 * n;
-        if (st == VG_OK) st = salloc((void **)&list, nsched * M * sizeof(uint32_t), s);
-        if (st == VG_OK)
-            st = salloc((void **)&lstart, slices * (kChainWaves + 1) * sizeof(uint32_t), s);
         if (st == VG_OK)
             st = launch("vg_pse_schedule", k_pse_lists, dim3(slices), dim3(kChainThreads), 0, s,
                         steps, M, (const uint32_t *)perm, (const uint32_t *)wstart, list, lstart);
@@ -1330,9 +1339,8 @@ vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const 
                         tv.sorted_idx, (const float *)angvel, ang_stride, birth, birth_stride, n,
                         w3, alive);
         if (st == VG_OK)
-            st = launch("vg_pse_fractions", k_pse_fractions,
-                        dim3(ceil_div(cells, 4)), dim3(256), 0, s, a, (uint32_t)cells, (const float *)alive, (const uint32_t *)foff,
-                        frac);
+            st = launch("vg_pse_fractions", k_pse_fractions, dim3(ceil_div(cells, 4)), dim3(256), 0, s,
+                        a, (uint32_t)cells, (const float *)alive, (const uint32_t *)foff, frac);
         const uint32_t buf_floats = kBufFront + (((uint32_t)totals[1] + 3u) & ~3u) + kBufBack;
         size_t lds = kChainWaves * buf_floats * sizeof(float);
         const bool resident = lds + totals[2] * sizeof(float) <= kLdsBytes;
@@ -1389,16 +1397,10 @@ vg_status pse_diffuse(const vg_tree *t, float *angvel, size_t ang_stride, const 
             st = launch("vg_pse_scatter", k_pse_scatter, dim3(ceil_div(n, 256)), dim3(256), 0, s,
                         tv.sorted_idx, (const float4 *)w, n, angvel, ang_stride);
     }
-    if (perm) sfree(perm, s);
-    if (wstart) sfree(wstart, s);
-    if (list) sfree(list, s);
-    if (lstart) sfree(lstart, s);
-    if (wide) sfree(wide, s);
-    if (frac) sfree(frac, s);
-    if (fsize) sfree(fsize, s);
-    if (foff) sfree(foff, s);
-    if (stmp) sfree(stmp, s);
-    if (dtot) sfree(dtot, s);
+    sfree(sched, s);
+    sfree(wide, s);
+    sfree(frac, s);
+    sfree(sizes, s);
     sfree(w, s);
     return st;
 }
