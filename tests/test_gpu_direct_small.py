@@ -60,3 +60,51 @@ def test_partials_of_many_tiles(vg, oracle, partials):
     assert np.linalg.norm(out.numpy() - want) <= 1e-5 * np.linalg.norm(want)
     # 2000 partials: 75 us with 16 loads under way, 480 with one
     assert ms < 0.2
+
+
+def _sum(vg, v, q, nq, out, stride):
+    """The kernels of a sum."""
+    vg.profile_reset()
+    vg.profile_enable(True)
+    try:
+        vg.direct_velocity(v, q, nq, out, 1.3, 0.7, 1, q_stride=stride)
+        vg.synchronize()
+        return set(vg.profile_dump())
+    finally:
+        vg.profile_enable(False)
+
+
+@pytest.mark.parametrize("n,nq", [(1, 1), (200, 20000), (256, 130), (300, 140000), (257, 300)])
+def test_one_share_of_the_sources_goes_out_directly(vg, oracle, n, nq):
+    """One launch where the sources are not split, several where they are; an
+    output that holds the vortons, or the queries at another stride, is written
+    once all have been read, to the same bits."""
+    print(f"[case] direct sum, {n} vortons at {nq} points, outputs among the inputs", flush=True)
+    rng = np.random.default_rng(n + nq)
+    pos, om, q = (rng.normal(size=(k, 3)).astype(F32) for k in (n, n, nq))
+    dp, dw, dq = (vg.DeviceArray.from_numpy(a) for a in (pos, om, q))
+    v = vg.vortons_view(dp, dw, n, uniform_size=0.2)
+    out = vg.DeviceArray.zeros((nq, 3))
+    split = n > 256 and nq < 131000
+    assert ("vg_direct_reduce" in _sum(vg, v, dq, nq, out, 3)) == split
+    got = out.numpy()
+    want = oracle.direct_velocity(pos, om, np.full(n, 0.2, F32), q, 1.3, 0.7, policy=1, threads=8)
+    assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+    # the vortons within the output, first as positions, then as vorticities
+    for field in (0, 1):
+        whole = rng.normal(size=(max(n, nq), 3)).astype(F32)
+        whole[:n] = (pos, om)[field]
+        both = vg.DeviceArray.from_numpy(whole)
+        u = vg.vortons_view(both, dw, n, uniform_size=0.2) if field == 0 else \
+            vg.vortons_view(dp, both, n, uniform_size=0.2)
+        assert "vg_direct_reduce" in _sum(vg, u, dq, nq, both, 3)
+        assert np.array_equal(both.numpy()[:nq], got)
+    # the queries' own places, and other ones
+    same = vg.DeviceArray.from_numpy(q)
+    assert ("vg_direct_reduce" in _sum(vg, v, same, nq, same, 3)) == split
+    assert np.array_equal(same.numpy(), got)
+    wide = np.zeros((nq, 5), F32)
+    wide[:, :3] = q
+    apart = vg.DeviceArray.from_numpy(wide)
+    assert "vg_direct_reduce" in _sum(vg, v, apart, nq, apart, 5)
+    assert np.array_equal(apart.numpy().ravel()[:3 * nq].reshape(nq, 3), got)

@@ -139,14 +139,19 @@ __global__ __launch_bounds__(kBlock) void k_direct(const float4 *__restrict__ A,
 // LDS at the end, so a block is 128 queries by one tile: 4096 queries of 4096
 // vortons make 512 workgroups instead of 32 (111 -> 22 us with the launches
 // around it).  Sources are prepared as they are staged, which spares the
-// packing launch.  Writes partials only: the reduction's launch orders them
-// after every read of the vortons, as the packed copy does above.
+// packing launch.  Several shares of the sources, or an `out` that may hold
+// vortons or other queries, go through partials: the reduction's launch orders
+// them after every read, as the packed copy does above for the vortons.  Otherwise (partial
+// null) the sums go out as the reduction of one partial gives them: 100
+// vortons at 400,000 points and a wait, 55 us by the blocks above, 80 with a
+// partial (its allocation and a launch more), 51 without.
 constexpr int kSmallQPT = 2, kSmallQueries = 64 * kSmallQPT;
 
 template <int POLICY, int VECPOT, int GRID>
 __global__ __launch_bounds__(kBlock) void k_direct_small(SourceView sv, size_t n, float spread,
-                                                         size_t chunk, QueryView qv,
-                                                         float *__restrict__ partial) {
+                                                         size_t chunk, QueryView qv, float circ,
+                                                         float *__restrict__ partial,
+                                                         float *out) {
     __shared__ float4 sA[kTile], sB[kTile];
     __shared__ float share[4][3 * kSmallQueries];
     const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
@@ -199,10 +204,12 @@ __global__ __launch_bounds__(kBlock) void k_direct_small(SourceView sv, size_t n
     }
     __syncthreads();
     const size_t first = 3 * (size_t)blockIdx.x * kSmallQueries;
-    for (int i = (int)threadIdx.x; i < 3 * kSmallQueries; i += kBlock)
-        if (first + i < 3 * qv.nq)
-            partial[(size_t)blockIdx.y * 3 * qv.nq + first + i] =
-                (share[0][i] + share[1][i]) + (share[2][i] + share[3][i]);
+    for (int i = (int)threadIdx.x; i < 3 * kSmallQueries; i += kBlock) {
+        if (first + i >= 3 * qv.nq) break;
+        const float v = (share[0][i] + share[1][i]) + (share[2][i] + share[3][i]);
+        if (partial) partial[(size_t)blockIdx.y * 3 * qv.nq + first + i] = v;
+        else out[first + i] = (0.f + v) * circ;
+    }
 }
 
 // Fixed-order Kahan reduction of the source-split partials, kReduceAhead of
@@ -310,6 +317,19 @@ struct Scratch {
     size_t bytes = 0;
 };
 
+// Whether a workgroup's results may lie where another still reads: out's
+// floats among the vortons', or among the queries' but in their own places.
+bool may_overlap(const vg_vortons *v, const QueryView &qv, const float *out) {
+    const uintptr_t o0 = (uintptr_t)out, o1 = o0 + 3 * qv.nq * sizeof(float);
+    auto meets = [&](const float *p, size_t n, size_t stride, size_t width) {
+        const uintptr_t p0 = (uintptr_t)p;
+        return p && p0 < o1 && o0 < p0 + ((n - 1) * stride + width) * sizeof(float);
+    };
+    return meets(v->pos, v->n, v->stride, 3) || meets(v->angvel, v->n, v->stride, 3) ||
+           meets(v->size, v->n, v->stride, 1) ||
+           (!(qv.q == out && qv.stride == 3) && meets(qv.q, qv.nq, qv.stride, 3));
+}
+
 inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
 template <int VECPOT, int GRID>
@@ -347,8 +367,13 @@ vg_status run_direct(const vg_vortons *v, QueryView qv, float spread, float circ
     bool small = false;
     const size_t split_queries = ceil_div(qv.nq, (size_t)kSmallQueries);
     if ((size_t)qblocks * nsplit < 1024) {
+        // 2048 workgroups, or one share of two tiles where the queries alone make
+        // half as many (300 vortons at 200,000 points and a wait: 58 against 75
+        // us in two shares; 2,000 vortons: 252 and, without the allocation, 230)
         const size_t tiles = ceil_div(n, (size_t)kTile);
-        const size_t want = (2048 + split_queries - 1) / split_queries;
+        const size_t want = split_queries >= 1024 && tiles <= 2
+                                ? 1
+                                : (2048 + split_queries - 1) / split_queries;
         const size_t per = (tiles + std::min(tiles, want) - 1) / std::min(tiles, want);
         const size_t ns = (tiles + per - 1) / per, bytes = ns * qv.nq * 3 * sizeof(float);
         if (ns < 65536 && 2 * align256(src_bytes) + align256(std::max(bytes, part_bytes)) <=
@@ -356,7 +381,7 @@ vg_status run_direct(const vg_vortons *v, QueryView qv, float spread, float circ
             small = true;
             chunk = per * kTile;
             nsplit = (uint32_t)ns;
-            part_bytes = bytes;
+            part_bytes = ns > 1 || may_overlap(v, qv, out) ? bytes : 0;
         }
     }
     float4 *A = nullptr, *B = nullptr;
@@ -386,8 +411,8 @@ vg_status run_direct(const vg_vortons *v, QueryView qv, float spread, float circ
                         ? k_direct_small<VG_RSQRT_REFERENCE, VECPOT, GRID>
                         : k_direct_small<VG_RSQRT_ACCURATE, VECPOT, GRID>;
         vg_status st = launch(name, kern, dim3((uint32_t)split_queries, nsplit), dim3(kBlock), 0, s,
-                              source_view(v), n, spread, chunk, qv, partial);
-        if (st == VG_OK)
+                              source_view(v), n, spread, chunk, qv, circ, partial, out);
+        if (st == VG_OK && partial)
             st = launch("vg_direct_reduce", k_reduce_split, dim3(ceil_div(qv.nq, 256)), dim3(256),
                         0, s, (const float *)partial, nsplit, qv.nq, circ, out);
         if (!fixed.base) sfree(partial, s);
