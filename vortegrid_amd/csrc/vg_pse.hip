@@ -62,7 +62,7 @@ vg_status tree_checked_view(const vg_tree *t, TreeView *v);
 namespace {
 
 constexpr int kPseThreads = 512;     // k_pse_phase
-constexpr int kChainThreads = 1024;  // k_pse_phase_chain (512: 4.5 against 4.0 ms)
+constexpr int kChainThreads = 1024;  // k_pse_phase_chain (512: 4.5 against 4.0 ms, with the stretching)
 constexpr int kPseWaves = kPseThreads / 64, kChainWaves = kChainThreads / 64;
 // Vortons of a cell and its 7 forward cells that the chain's LDS buffers hold
 // (16 waves share 160 KB); 1M vortons at 129^3 have at most 442.
@@ -656,7 +656,8 @@ __global__ __launch_bounds__(256) void k_pse_fractions(PseArgs a, uint32_t cells
 }
 
 // Groups of four steps whose fractions a lane holds ahead of their use
-// (4, 6 and 8 groups: 3.88, 3.90 and 4.00 ms for the call at 1M vortons).
+// (4, 6 and 8 groups: 3.88, 3.90 and 4.00 ms for the vorticity update, this
+// call and the stretching, at 1M vortons).
 constexpr int kRing = 4;
 
 // A cell as the chain takes it: its partners and its fractions.
@@ -973,7 +974,8 @@ __global__ __launch_bounds__(kChainThreads) void k_pse_lists(uint32_t steps, uin
 // current one runs.
 // RESIDENT: the component of both slices' vortons stays in LDS for the whole
 // phase (`buf_floats` per wave, then the values), so a step waits for no
-// global load or store: 3.88 against 4.10 ms for the call at 1M vortons.
+// global load or store: 3.88 against 4.10 ms for the vorticity update at 1M
+// vortons.
 // Otherwise (slices too full for the LDS) they stay in w3.
 template <bool RESIDENT>
 __global__ __launch_bounds__(kChainThreads) void k_pse_phase_chain(

@@ -439,10 +439,11 @@ __global__ void k_aggregate_views(const TreeView *__restrict__ views, uint32_t l
 // One tree's layers of at most kTopPoints points, in one workgroup with a
 // barrier between layers: each is a single trip of it, all latency, and as
 // launches of one stream they took 5 us each (a tree of 4,096 vortons, whose
-// layers from 9x9x9 up are four launches: a frame 366 -> 355 us).  Batched
-// trees keep a launch per layer: those are replayed from a graph, where the
-// chain in one workgroup gained nothing on one tree of 65,536 vortons (176.6
-// against 178.3 us a frame) and lost on 256 trees (3.45 against 3.59 ms).
+// layers from 9x9x9 up are four launches: a frame 366 -> 355 us; each layer
+// still goes out to memory and back).  Batched trees keep a launch per layer:
+// the chain in one workgroup gained nothing on one tree of 65,536 vortons
+// (176.6 against 178.3 us a frame of plain launches) and lost on 256 trees
+// replayed from a graph (3.45 against 3.59 ms).
 constexpr size_t kTopPoints = 1024;
 struct TopLayers {
     Nested ng;
