@@ -27,11 +27,13 @@
 // LDS return path 40 of the CU's cycles per 64 interactions, more than their
 // arithmetic: 3.0 ms for the 1M-vorton walk (129^3 points, near_k 3) and 3.5
 // ms for 256 effects of 33^3 (near_k 2).  With four they take 10 and the walk
-// is bound by VALU issue (23 operations per far interaction, about 3 cycles
-// each at the four waves per SIMD that its 101 registers allow): 1.89 and 2.5
-// ms.  Capping the registers at 96 or 80 for more waves was slower (2.9 ms
+// is bound by VALU issue: 1.17e9 VALU instructions a launch, 4 cycles of a
+// SIMD each, are 1.91 ms at 2.4 GHz, the LDS path 0.8: 1.89 and 2.5 ms.
+// Capping the 101 registers at 96 or 80 for more waves was slower (2.9 ms
 // against 2.7 for the whole frame): the four points' interleaved chains hide
-// latency better than more waves do.
+// latency better than more waves do.  Grids of 1 to 3 points on two axes, whose
+// layers hold a few clusters each, were up to a tenth faster with one point per
+// lane (3x3x513, near_k 1: 37.8 against 42.7 us).
 #include "vg_internal.h"
 
 namespace vg {
